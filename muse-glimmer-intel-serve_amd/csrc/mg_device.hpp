@@ -431,6 +431,14 @@ namespace mg
     {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
     }
+    // v_mfma_f32_32x32x16_bf16: lane l = 32h + n holds row n of A (column n of
+    // B) and its k-elements 8h..8h+7; C lane l holds rows 8 (r / 4) + 4h + r % 4
+    // of column n, r = 0..15
+    typedef float f32x16 __attribute__((ext_vector_type(16)));
+    MG_DEV f32x16 mfma_bf16_32(bf16x8 a, bf16x8 b, f32x16 c)
+    {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+    }
     MG_DEV bf16x8 ld_bf16x8(const uint16_t *p)
     {
         return __builtin_bit_cast(bf16x8, *reinterpret_cast<const Vec<uint32_t, 4> *>(p));

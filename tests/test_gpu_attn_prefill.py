@@ -142,3 +142,40 @@ def test_errors(prims):
     q = torch.zeros((20, 8, 128), dtype=torch.bfloat16, device="cuda:0")
     with pytest.raises(Exception, match="cache ring"):
         prims.attn_prefill(q, kc, kc, 0, 0.1)
+
+
+@pytest.mark.parametrize("T,nq,nkv,D,pos0,window", (
+    (1, 40, 8, 128, 4000, 0),       # one row: eleven live pairs short of one wave, many parts
+    (2, 7, 7, 64, 9000, 0),         # more parts than one wave merges
+    (51, 40, 8, 128, 2111, 0),      # 255 pairs: a tile one pair short of full
+    (52, 40, 8, 128, 2112, 0),      # 260 pairs: a second tile of four
+    (33, 32, 2, 128, 5000, 0),      # two tiles of 16 heads a row, the last with one wave live
+    (129, 16, 2, 64, 1000, 700),    # window starts inside, before and past the parts
+    (300, 2, 2, 128, 5000, 2000),   # 256 rows a tile: parts whose keys lie before the last rows' windows
+    (400, 8, 1, 128, 0, 0),         # causal from key 0: tiles of different length, empty parts
+))
+def test_key_split(prims, T, nq, nkv, D, pos0, window):
+    """few pair tiles over many keys: the tiles' keys split into parts that a
+    second kernel merges; edges of pair tiles, parts and windows, on a ring
+    that has wrapped when a window allows it"""
+    slots = T + window + 40 if window else pos0 + T
+    rows = sorted({0, 1, T // 2, T - 2, T - 1} & set(range(T)))
+    prefill_case(prims, T, nq, nkv, D, slots, pos0, window=window, seed=180 + T, heads=(0, nq // 2, nq - 1), rows=rows)
+
+
+def test_key_split_without_workspace(prims):
+    """a context whose workspace holds no partials runs the tiles unsplit: the
+    same envelope, and both close to each other"""
+    import mgprims
+    import torch
+    small = mgprims.Prims(0, workspace_bytes=4096)
+    q = to_dev(O.normal(190, (20, 40, 128), 0.0, 1.0, BF16), BF16)
+    k = to_dev(O.normal(191, (3000, 8, 128), 0.0, 1.0, BF16), BF16)
+    v = to_dev(O.normal(192, (3000, 8, 128), 0.0, 1.0, BF16), BF16)
+    a = small.attn_prefill(q, k, v, 2980, 0.088)
+    b = prims.attn_prefill(q, k, v, 2980, 0.088)
+    small.close()
+    # both are within 2^-8 sum p |v| of the same value, and sum p |v| is below 1
+    assert float((a - b).abs().max()) <= 2 * TOL
+    prefill_case(prims, 20, 40, 8, 128, 3000, 2980, seed=190)
+    assert torch.isfinite(a).all()
