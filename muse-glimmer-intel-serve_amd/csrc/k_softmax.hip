@@ -16,8 +16,9 @@
 //
 // Rows of up to 2048 keys: one wave per row (the fast path runs one-wave
 // work-groups), the row in registers (8 keys per lane per chunk), one read
-// and one write of HBM. Longer rows (decode,
-// q = 1, k = 131072): split over work-groups of 4096 keys; pass A writes each
+// and one write of HBM; f32 scores to 16-bit probabilities of up to 16384 keys
+// the same with two to eight waves per row (k_softmax_group). Longer rows
+// (decode, q = 1, k = 131072): split over work-groups of 4096 keys; pass A writes each
 // chunk's (max, sum) partial, pass B merges the partials of its row in chunk
 // order (the k_attn_decode_combine rule, src/gpu/gpu_engine.cpp:1816-1857, with
 // the sum rescaled in f64), re-reads its chunk (an L2 hit: a chunk goes to the
@@ -72,11 +73,24 @@ namespace mg
         return float(mgm::tanh(double(s))) * cap;
     }
 
+    // the tanh table's copy in a wave's own LDS, made when its first key needs it
+    struct CapTab
+    {
+        double *tab; // 128 entries
+        bool have;
+    };
+
     // 8 raw f32 scores of a row -> capped scores (bit e of vis set: key e is
-    // visible, else it becomes -inf). Each key takes mgm::softcap_score_fast;
-    // the few it does not certify (|s / cap| >= 2^-5, or a rounding too close
-    // to call) are redone by the plain chain, behind one wave-uniform branch.
-    MG_DEV void cap8(const SmArgs &a, float *v, uint32_t vis)
+    // visible, else it becomes -inf). Each key takes mgm::softcap_score_fast.
+    // A wave with a key it does not certify (|s / cap| >= 2^-5, or a rounding
+    // too close to call) evaluates the tail's table polynomial for its keys, four
+    // side by side without a branch, and takes it where both ends of its error
+    // interval round to one f32 (tests/test_tanh_fast.py runs every f32 below 22);
+    // the rest (|s / cap| >= 1, inf, NaN, about 3 in 10^6 others) are redone by
+    // the plain chain. Bits are the twin's on every path. Scores of std 5 under
+    // a cap of 30 (most of them past 2^-5), [40, 2048, 2048]: 419 -> 219 us against
+    // the plain chain in the table's place.
+    MG_DEV void cap8(const SmArgs &a, float *v, uint32_t vis, CapTab &ct)
     {
         float x[8];
         uint32_t slow = 0;
@@ -90,9 +104,34 @@ namespace mg
             slow |= uint32_t(in && !ok) << e;
         }
         if (__builtin_amdgcn_ballot_w64(slow != 0u)) {
+            if (!ct.have) {
+                const int lane = threadIdx.x & 63;
+                *reinterpret_cast<Vec<double, 2> *>(ct.tab + 2 * lane) =
+                    *reinterpret_cast<const Vec<double, 2> *>(mgm::kTanhTab + 2 * lane);
+                wave_lds_sync();
+                ct.have = true;
+            }
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if ((slow >> e) & 1u) v[e] = capped_score_slow(x[e], a.scale, a.cap);
+            for (int g = 0; g < 8; g += 4) {
+#pragma unroll
+                for (int e = g; e < g + 4; ++e) {
+                    const float s = x[e] * a.scale, as = __builtin_fabsf(s);
+                    const float q = mgm::softcap_quotient(s, a.cap, a.rcap);
+                    const double aq = __builtin_fabs(double(q));
+                    double tl, tu;
+                    mgm::tanh_interval(mgm::tanh_table_abs(__builtin_fmin(aq, 0x1.fffffffffffffp-1), ct.tab), tl, tu);
+                    const float lo = float(tl);
+                    const bool ok = as > 0x1p-100f && as < 0x1p100f && aq < 1.0 && lo == float(tu);
+                    const bool take = ok && ((slow >> e) & 1u);
+                    v[e] = take ? __builtin_copysignf(lo, q) * a.cap : v[e];
+                    slow &= take ? ~(1u << e) : ~0u;
+                }
+            }
+            if (__builtin_amdgcn_ballot_w64(slow != 0u)) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if ((slow >> e) & 1u) v[e] = capped_score_slow(x[e], a.scale, a.cap);
+            }
         }
     }
 
@@ -240,16 +279,16 @@ namespace mg
     // With a softcap (CAP) each visible key first becomes the twin's capped
     // score, bit for bit (cap8: mgm::softcap_score_fast, and the plain chain
     // for the keys it does not certify), and c2 = log2 e.
-    // Key indices are 32-bit (rows of at most 2048 keys); chunks entirely
+    // Key indices are 32-bit; chunks entirely
     // visible skip the per-key mask, chunks entirely masked skip the
     // arithmetic and store zeros. A row whose sum is not finite (NaN or
     // infinite scores) is redone on the accurate path.
     //
-    // One row of the fast path in a wave's registers: lane `lane` holds keys
-    // 512 c + 8 lane + e, raw scores until fast_finish transforms them.
-    // key of element e of chunk c in lane `lane`: two runs of 4 keys, 256 apart,
-    // so each 16-byte load instruction of the wave covers 1 KiB contiguously
-    MG_DEV int fast_key(int c, int e, int lane) { return c * 512 + (e >> 2) * 256 + lane * 4 + (e & 3); }
+    // One row of the fast path in the registers of WPR waves: wave w takes the
+    // 512-key chunks w, w + WPR, ..., raw scores until fast_exp transforms them.
+    // key of element e in lane `lane` of the chunk at cb: two runs of 4 keys, 256
+    // apart, so each 16-byte load instruction of the wave covers 1 KiB contiguously
+    MG_DEV int fast_key(int cb, int e, int lane) { return cb + (e >> 2) * 256 + lane * 4 + (e & 3); }
 
     template <int CH>
     struct FastRow
@@ -260,15 +299,14 @@ namespace mg
     };
 
     // issue the loads of a row's visible 512-key chunks (nothing waits on them
-    // here; the finish waits for each chunk's own loads).
-    // VEC (rows of a multiple of 8 keys, 16-byte aligned): every lane issues
-    // its two 16-byte loads per chunk as raw buffer loads over the row's
-    // visible prefix [0, hi]; loads of keys past hi (and lanes wholly below lo,
-    // sent past the end) are out of range, return zeros and touch no memory.
-    // With no branch around them the compiler counts the loads exactly and a
-    // chunk waits only for its own data. Otherwise keys load one by one.
-    template <int CH, bool VEC>
-    MG_DEV void fast_load(const SmArgs &a, const float *__restrict__ x, int64_t row, int lane, FastRow<CH> &r)
+    // here; the finish waits for each chunk's own loads): every lane issues its
+    // two 16-byte loads per chunk as raw buffer loads over the row's visible
+    // prefix [0, hi]; loads of keys past hi (and lanes wholly below lo, sent past
+    // the end) are out of range, return zeros and touch no memory. With no branch
+    // around them the compiler counts the loads exactly and a chunk waits only
+    // for its own data. A row need only be aligned to its elements.
+    template <int CH, int WPR>
+    MG_DEV void fast_load(const SmArgs &a, const float *__restrict__ x, int64_t row, int lane, int w, FastRow<CH> &r)
     {
         // a row past the end gets the empty range, so its loads (out of
         // range) touch nothing; no branch, so the load count stays exact
@@ -276,65 +314,52 @@ namespace mg
         row_range(a, row, r.lo64, r.hi64);
         r.lo64 = r.live ? r.lo64 : 0;
         r.hi64 = r.live ? r.hi64 : -1;
-        const int lo = int(r.lo64), hi = int(r.hi64); // 0 <= lo <= kc, -1 <= hi < kc <= 2048
+        const int lo = int(r.lo64), hi = int(r.hi64); // 0 <= lo <= kc, -1 <= hi < kc <= 512 CH WPR
         const float *xr = x + row * a.ldx;
-        if constexpr (VEC) {
-            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-            // word 3 of a gfx9 raw buffer descriptor (32-bit data, no swizzle)
-            const __amdgpu_buffer_rsrc_t rs =
-                __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(xr), short(0), (hi + 1) * 4, 0x00020000);
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        // word 3 of a gfx9 raw buffer descriptor (32-bit data, no swizzle)
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(xr), short(0), (hi + 1) * 4, 0x00020000);
 #pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                const int ja = c * 512 + lane * 4, jb = ja + 256;
-                const int offa = ja + 3 >= lo ? ja * 4 : 0x40000000;
-                const int offb = jb + 3 >= lo ? jb * 4 : 0x40000000;
-                const u32x4 p = __builtin_amdgcn_raw_buffer_load_b128(rs, offa, 0, 2); // 2: non-temporal
-                const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(rs, offb, 0, 2);
-                // (element to a prvalue first: this clang lowers bit_cast of an
-                // ext_vector element lvalue to a read of element 0)
+        for (int c = 0; c < CH; ++c) {
+            const int ja = (c * WPR + w) * 512 + lane * 4, jb = ja + 256;
+            const int offa = ja + 3 >= lo ? ja * 4 : 0x40000000;
+            const int offb = jb + 3 >= lo ? jb * 4 : 0x40000000;
+            const u32x4 p = __builtin_amdgcn_raw_buffer_load_b128(rs, offa, 0, 2); // 2: non-temporal
+            const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(rs, offb, 0, 2);
+            // (element to a prvalue first: this clang lowers bit_cast of an
+            // ext_vector element lvalue to a read of element 0)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    r.v[c][e] = __builtin_bit_cast(float, uint32_t(p[e]));
-                    r.v[c][e + 4] = __builtin_bit_cast(float, uint32_t(q[e]));
-                }
-            }
-        } else {
-#pragma unroll
-            for (int c = 0; c < CH; ++c) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int j = fast_key(c, e, lane);
-                    r.v[c][e] = (j >= lo && j <= hi) ? xr[j] : 0.0f;
-                }
+            for (int e = 0; e < 4; ++e) {
+                r.v[c][e] = __builtin_bit_cast(float, uint32_t(p[e]));
+                r.v[c][e + 4] = __builtin_bit_cast(float, uint32_t(q[e]));
             }
         }
     }
 
-    // transform, normalise and store a loaded row; returns true (nothing
-    // stored) for a row whose sum is not finite (NaN or infinite scores),
-    // which the caller redoes on the accurate path
-    template <class SO, int CH, bool CAP>
-    MG_DEV bool fast_finish(const SmArgs &a, typename SO::raw *__restrict__ y, int64_t row, float c2, bool vec,
-                            int lane, FastRow<CH> &r)
+    // the wave's share of a loaded row: scores (capped, masked) to 2^(s c2 - mc),
+    // mc = the wave's maximum times c2 (rounded); returns the maximum (-inf: no
+    // key with a weight) and the wave's sum
+    template <int CH, int WPR, bool CAP>
+    MG_DEV float fast_exp(const SmArgs &a, float c2, int lane, int w, FastRow<CH> &r, float &sum, double *tab)
     {
-        using ro = typename SO::raw;
-        if (!r.live) return false;
-        const int kc = int(a.kc), lo = int(r.lo64), hi = int(r.hi64);
+        [[maybe_unused]] CapTab ct{tab, false};
+        const int lo = int(r.lo64), hi = int(r.hi64);
         float m = kNegInf;
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
-            const int cb = c * 512;
+            const int cb = (c * WPR + w) * 512;
             if (cb > hi || cb + 511 < lo) continue;
             if (cb >= lo && cb + 511 <= hi) {
-                if constexpr (CAP) cap8(a, r.v[c], 0xffu);
+                if constexpr (CAP) cap8(a, r.v[c], 0xffu, ct);
             } else {
                 // a row without visible keys (lo = 0, hi = -1, mask_range)
                 // skipped every chunk above, so here 0 <= hi - lo < kc
                 uint32_t vis = 0;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) vis |= uint32_t(unsigned(fast_key(c, e, lane) - lo) <= unsigned(hi - lo)) << e;
+                for (int e = 0; e < 8; ++e) vis |= uint32_t(unsigned(fast_key(cb, e, lane) - lo) <= unsigned(hi - lo)) << e;
                 if constexpr (CAP) {
-                    cap8(a, r.v[c], vis);
+                    cap8(a, r.v[c], vis, ct);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) r.v[c][e] = (vis >> e) & 1u ? r.v[c][e] : kNegInf;
@@ -344,12 +369,12 @@ namespace mg
             for (int e = 0; e < 8; ++e) m = __builtin_fmaxf(m, r.v[c][e]);
         }
         m = dpp_max(m);
-        float sum = 0.0f;
+        sum = 0.0f;
         if (m != kNegInf) {
             const float mc = m * c2;
 #pragma unroll
             for (int c = 0; c < CH; ++c) {
-                const int cb = c * 512;
+                const int cb = (c * WPR + w) * 512;
                 if (cb > hi || cb + 511 < lo) continue;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
@@ -359,25 +384,37 @@ namespace mg
             }
         }
         sum = dpp_sum_f32(sum);
+        return m;
+    }
+
+    // the wave's share of the row times `f` to storage; chunks without a visible
+    // key, and all of them when `empty`, as zeros
+    typedef uint32_t u32x2u __attribute__((ext_vector_type(2), aligned(2)));
+    template <class SO, int CH, int WPR, bool VEC>
+    MG_DEV void fast_store(const SmArgs &a, typename SO::raw *__restrict__ y, int64_t row, float f, bool empty, int lane,
+                           int w, const FastRow<CH> &r)
+    {
+        using ro = typename SO::raw;
+        const int kc = int(a.kc), lo = int(r.lo64), hi = int(r.hi64);
         ro *yr = y + row * a.ldy;
-        if (m != kNegInf && !(sum < __builtin_huge_valf())) return true; // NaN / infinite scores
-        const float inv = m == kNegInf ? 0.0f : __builtin_amdgcn_rcpf(sum);
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
-            const int cb = c * 512;
-            const bool none = m == kNegInf || cb > hi || cb + 511 < lo;
+            const int cb = (c * WPR + w) * 512;
+            const bool none = empty || cb > hi || cb + 511 < lo;
 #pragma unroll
             for (int hh = 0; hh < 2; ++hh) {
                 const int j0 = cb + hh * 256 + lane * 4;
                 if (j0 >= kc) continue;
                 Vec<ro, 4> o;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o.v[e] = none ? ro(0) : SO::enc_finite(r.v[c][4 * hh + e] * inv);
-                if (vec && j0 + 4 <= kc) {
-                    const Vec<uint32_t, 2> u = __builtin_bit_cast(Vec<uint32_t, 2>, o);
+                for (int e = 0; e < 4; ++e) o.v[e] = none ? ro(0) : SO::enc_finite(r.v[c][4 * hh + e] * f);
+                const Vec<uint32_t, 2> u = __builtin_bit_cast(Vec<uint32_t, 2>, o);
+                if (VEC) {
                     uint32_t *q = reinterpret_cast<uint32_t *>(yr + j0);
                     __builtin_nontemporal_store(u.v[0], q);
                     __builtin_nontemporal_store(u.v[1], q + 1);
+                } else if (j0 + 4 <= kc) {
+                    *reinterpret_cast<u32x2u *>(yr + j0) = u32x2u{u.v[0], u.v[1]};
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
@@ -385,7 +422,6 @@ namespace mg
                 }
             }
         }
-        return false;
     }
 
     // One row per one-wave work-group. All of the row's loads are issued
@@ -397,10 +433,64 @@ namespace mg
         const int lane = threadIdx.x & 63;
         const int64_t row = blockIdx.x;
         FastRow<CH> r;
-        fast_load<CH, VEC>(a, x, row, lane, r);
+        fast_load<CH, 1>(a, x, row, lane, 0, r);
+        if (!r.live) return;
+        __shared__ double tab[CAP ? 128 : 1];
+        float sum;
+        const float m = fast_exp<CH, 1, CAP>(a, c2, lane, 0, r, sum, tab);
         // a row with non-finite sums is redone on the accurate path
-        if (fast_finish<SO, CH, CAP>(a, y, row, c2, VEC, lane, r))
+        if (m != kNegInf && !(sum < __builtin_huge_valf())) {
             softmax_row_accurate<SF32, SO, CH, CAP>(a, x + row * a.ldx, y + row * a.ldy, r.lo64, r.hi64, VEC, lane);
+            return;
+        }
+        fast_store<SO, CH, 1, VEC>(a, y, row, m == kNegInf ? 0.0f : __builtin_amdgcn_rcpf(sum), m == kNegInf, lane, 0, r);
+    }
+
+    // Rows of 2049..16384 keys, one per work-group of WPR waves with the row in
+    // their registers: one read and one write of HBM, where the split passes
+    // below read the scores twice (40 heads of 1000 queries over 4000 keys: 254 ->
+    // 143 us, 6.2 TB/s of the visible scores and the probabilities; 40 decode rows
+    // of 16384: 11.3 -> 7.4, a launch less). Bound by HBM. Each wave takes its own maximum and sum;
+    // the waves meet once, in LDS, and the move to the row's maximum goes into
+    // each wave's factor: 2^(mc_w - mc) / L, from the rounded maxima mc the
+    // exponents used, so their roundings cancel as within one wave.
+    // A row with NaN or infinite scores gets NaN at every visible key (its sum
+    // is NaN) and zeros at the masked ones, as in the split passes.
+    template <class SO, int WPR, bool CAP, bool VEC>
+    __global__ __launch_bounds__(64 * WPR) void k_softmax_group(const float *__restrict__ x,
+                                                                typename SO::raw *__restrict__ y, SmArgs a, float c2)
+    {
+        using ro = typename SO::raw;
+        constexpr int CH = 4;
+        __shared__ float red[2 * WPR];
+        const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+        const int64_t row = blockIdx.x;
+        FastRow<CH> r;
+        fast_load<CH, WPR>(a, x, row, lane, w, r);
+        __shared__ double tab[CAP ? 128 * WPR : 1];
+        float sum;
+        const float m = fast_exp<CH, WPR, CAP>(a, c2, lane, w, r, sum, tab + (CAP ? 128 * w : 0));
+        if (lane == 0) {
+            red[w] = m;
+            red[WPR + w] = sum;
+        }
+        __syncthreads();
+        float M = red[0];
+#pragma unroll
+        for (int i = 1; i < WPR; ++i) M = __builtin_fmaxf(M, red[i]);
+        const float Mc = M * c2;
+        float L = 0.0f;
+#pragma unroll
+        for (int i = 0; i < WPR; ++i)
+            if (red[i] != kNegInf) L += red[WPR + i] * __builtin_amdgcn_exp2f(red[i] * c2 - Mc);
+        if (M != kNegInf && !(L < __builtin_huge_valf())) {
+            ro *yr = y + row * a.ldy;
+            for (int j = int(threadIdx.x); j < int(a.kc); j += 64 * WPR)
+                yr[j] = j >= int(r.lo64) && j <= int(r.hi64) ? SO::enc32(__builtin_nanf("")) : ro(0);
+            return;
+        }
+        const float f = m == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(m * c2 - Mc) * __builtin_amdgcn_rcpf(L);
+        fast_store<SO, CH, WPR, VEC>(a, y, row, f, m == kNegInf, lane, w, r);
     }
 
     // ------------------------------------------------------------- split rows
@@ -722,13 +812,13 @@ namespace mg
         const bool vec = a.kc % 8 == 0 && a.ldx % 8 == 0 && a.ldy % 8 == 0 && aligned16(x) && aligned16(y);
         const ri *xi = static_cast<const ri *>(x);
         ro *yo = static_cast<ro *>(y);
+        // the fast capped score takes 1 <= |cap| <= 2^20 (mg_softcap_fast.hpp,
+        // the range its host checker sweeps); other caps take the accurate kernel
+        const float acap = __builtin_fabsf(a.cap);
+        [[maybe_unused]] const bool cap_ok = !CAP || (acap >= 1.0f && acap <= 0x1p20f);
         if (a.kc <= 2048) {
             const unsigned blocks = unsigned((a.nrows + 3) / 4);
             need(a.nrows < (int64_t(1) << 31), "softmax: too many rows");
-            // the fast capped score takes 1 <= |cap| <= 2^20 (mg_softcap_fast.hpp,
-            // the range its host checker sweeps); other caps take the accurate kernel
-            const float acap = __builtin_fabsf(a.cap);
-            const bool cap_ok = !CAP || (acap >= 1.0f && acap <= 0x1p20f);
             if constexpr (SI::dt == F32 && sizeof(ro) == 2) if (cap_ok && (CAP || a.scale > 0.0)) {
                 // log2-domain factor: the scale folds in unless the cap comes after it
                 const float c2 = float((CAP ? 1.0 : double(a.scale)) * 1.4426950408889634);
@@ -767,6 +857,31 @@ namespace mg
              "softmax: partials exceed the context workspace (raise workspace_bytes at mg_open)");
         float2 *part = static_cast<float2 *>(c->work);
         const dim3 grid{unsigned(nch), unsigned(a.nrows), 1u};
+        // rows that fit one work-group's registers: every row count (a decode
+        // step's 40 rows too: one launch instead of two)
+        if constexpr (SI::dt == F32 && sizeof(ro) == 2)
+            if (a.kc <= 16384 && cap_ok && (CAP || a.scale > 0.0)) {
+                const float c2 = float((CAP ? 1.0 : double(a.scale)) * 1.4426950408889634);
+                // as in k_softmax_fast, a reserved and untouched part of the LDS
+                // holds the waves per SIMD where the row streams best: 4 for
+                // vector rows of two waves (40 000 rows of 4000: 143 us against
+                // 161 unheld, 150 at 5, 159 at 6), 6 for the others (10 000 of
+                // 16 000: 158 against 162, 159 at 4; 28 000 of 5003: 145 against
+                // 149, 155 at 4)
+                auto go = [&](auto kern, unsigned waves) {
+                    const unsigned hold = vec && waves == 2 ? 4u : 6u;
+                    const unsigned lds = CAP ? 0u : (kLdsPerCu - 8192u) * waves / (4u * hold);
+                    hipLaunchKernelGGL(kern, dim3(unsigned(a.nrows)), dim3(64 * waves), lds, c->stream, xi, yo, a, c2);
+                };
+                if (a.kc <= 4096)
+                    vec ? go(k_softmax_group<SO, 2, CAP, true>, 2) : go(k_softmax_group<SO, 2, CAP, false>, 2);
+                else if (a.kc <= 8192)
+                    vec ? go(k_softmax_group<SO, 4, CAP, true>, 4) : go(k_softmax_group<SO, 4, CAP, false>, 4);
+                else
+                    vec ? go(k_softmax_group<SO, 8, CAP, true>, 8) : go(k_softmax_group<SO, 8, CAP, false>, 8);
+                check_launch("k_softmax_group");
+                return;
+            }
         if constexpr (SI::dt == F32 && sizeof(ro) == 2 && !CAP) {
             const float c2 = float(double(a.scale) * 1.4426950408889634);
             if (vec && a.kc < (int64_t(1) << 28)) {

@@ -262,3 +262,59 @@ def test_errors(prims):
     xb = torch.zeros((1, 1, 64), dtype=torch.bfloat16, device="cuda:0")
     with pytest.raises(mgprims.MgError, match="input dtype"):
         prims.softmax_rows(xb, y, 1.0, f32_compat=True)
+
+
+@pytest.mark.parametrize("dt_out", (BF16, F16))
+@pytest.mark.parametrize("kc", (2049, 2056, 2731, 4096, 4097, 8192, 8195, 16384))
+@pytest.mark.parametrize("mask,window", ((O.MASK_CAUSAL, 0), (O.MASK_WINDOW, 700)))
+def test_group_rows(prims, kc, dt_out, mask, window):
+    """rows of one work-group's registers (2049..16384 keys): both ends of each
+    wave count, odd lengths (rows aligned to their elements only), rows that end
+    in every wave's share and windows that leave some waves no key"""
+    q = 24
+    for q_pos0 in (kc - q, kc // 2, 0):
+        y, ref = run(prims, 2, q, kc, dt_out=dt_out, mask=mask, window=window, q_pos0=q_pos0)
+        check(y, ref, dt_out, visible(2, q, kc, mask, window, q_pos0))
+
+
+@pytest.mark.parametrize("kc", (2500, 5003, 16383))
+def test_group_rows_softcap(prims, kc):
+    y, ref = run(prims, 2, 24, kc, softcap=30.0, std=60.0, q_pos0=kc - 24)
+    check(y, ref, BF16, visible(2, 24, kc, O.MASK_CAUSAL, 0, kc - 24))
+
+
+@pytest.mark.parametrize("kc", (3, 509, 1023, 2047))
+def test_short_odd_rows(prims, kc):
+    """rows of odd length through the vector accesses of the one-wave kernel"""
+    q = min(kc, 16)
+    y, ref = run(prims, 3, q, kc, q_pos0=kc - q)
+    check(y, ref, BF16, visible(3, q, kc, O.MASK_CAUSAL, 0, kc - q))
+
+
+@pytest.mark.parametrize("kc", (3001, 4096, 10000))
+def test_group_rows_nonfinite(prims, kc):
+    """a NaN or +inf score makes every visible probability NaN and leaves the
+    masked ones 0; rows of -inf scores only are all 0; the rows beside them
+    are untouched"""
+    import torch
+    q = 8
+    x = O.to_f64(O.normal(14, (1, q, kc), 0.0, 3.0, F32), F32).astype(np.float32)
+    x[0, 1, 5] = np.nan
+    x[0, 2, kc // 2] = np.inf
+    x[0, 3, :] = -np.inf
+    x[0, 4, 10:200] = -np.inf
+    dx = torch.from_numpy(x).cuda()
+    dy = torch.full((1, q, kc), 7.0, dtype=torch.bfloat16, device="cuda:0")
+    q_pos0 = kc - q - 100
+    prims.softmax_rows(dx, dy, SCALE, O.MASK_CAUSAL, 0, q_pos0)
+    y = dy.float().cpu().numpy()
+    vis = visible(1, q, kc, O.MASK_CAUSAL, 0, q_pos0)
+    assert np.all(y[~vis] == 0.0)
+    for r in (1, 2):
+        assert np.all(np.isnan(y[0, r][vis[0, r]])), r
+    assert np.all(y[0, 3] == 0.0)
+    for r in (0, 4, 5, 6, 7):
+        xr = x[0, r].astype(np.float64) * np.float32(SCALE)
+        e = np.where(vis[0, r], np.exp(xr - xr[vis[0, r]].max()), 0.0)
+        d = ulp_diff16(O.from_f64(y[0, r].astype(np.float64), BF16), O.from_f64(e / e.sum(), BF16))
+        assert d.max() <= 1, r
