@@ -273,6 +273,133 @@ namespace mg
         }
     }
 
+    // Two to eight activation rows over a weight of 256-quant rows: the weights
+    // are read and dequantized once for all of them, and the products run on the
+    // matrix cores (v_mfma_f32_16x16x32_bf16: A = 16 weight rows, B = the batch
+    // padded to 16 columns by its last row, whose columns are not stored). The
+    // vector form above spends a dot instruction and two 16-byte activation loads
+    // per lane for every batch row, and takes the weights twice past four rows.
+    // A work-group of NW waves serves 16 RT weight rows; its waves take 256-quant
+    // pieces of the rows in turn, the next piece in flight while the current one
+    // is dequantized, and their sums meet in LDS in wave order. A lane's 16
+    // quants are the k-elements of two products (quants 16 c + 8 i .. of the 64 for
+    // product i, of the activations alike).
+    // [6656, 19968], 6 rows: 108 -> 34 us (4.2 TB/s); [25600, 5120], 8 rows: 116 -> 36,
+    // 2 rows: 35 -> 32. Bound by the weight stream (its own probe: 22 us) and the
+    // activations' way through the L1 (1 KiB a load and wave, twice the weights').
+    template <int RT, int NW>
+    __global__ __launch_bounds__(64 * NW) void k_gemv_q8_0_mfma(const int8_t *__restrict__ W,
+                                                               const uint16_t *__restrict__ D,
+                                                               const uint16_t *__restrict__ X, float *__restrict__ Y,
+                                                               int64_t in, int64_t out, int64_t ldx, int64_t ldy, int B)
+    {
+        // each wave's piece, row pitch 272 bytes: a piece is loaded 256 contiguous
+        // bytes a row (64 a row and load straight in the operand's layout ran
+        // slower) and read back 16 rows at a time without bank conflicts
+        constexpr int PITCH = 272;
+        __shared__ __align__(16) char lw[NW][RT * 16 * PITCH];
+        const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+        const int n = lane & 15, c = lane >> 4;
+        const int64_t r0 = int64_t(blockIdx.x) * (16 * RT);
+        const uint16_t *dp[RT];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const int64_t r = r0 + 16 * t + n, row = r < out ? r : out - 1;
+            dp[t] = D + row * (in / 32);
+        }
+        const int8_t *wq[RT][4];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int64_t r = r0 + 16 * t + 4 * s + c, row = r < out ? r : out - 1;
+                wq[t][s] = W + row * in + 16 * n;
+            }
+        char *lb = lw[wv];
+        const uint16_t *xp = X + int64_t(n < B ? n : B - 1) * ldx + 16 * c;
+        const int np = int(in / 256);
+        Vec<uint32_t, 4> w[RT][4], d[RT];
+        auto load = [&](int m) {
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    w[t][s] = ld16_stream<uint32_t, 4>(reinterpret_cast<const uint32_t *>(wq[t][s] + 256 * int64_t(m)));
+                d[t] = *reinterpret_cast<const Vec<uint32_t, 4> *>(dp[t] + 8 * int64_t(m));
+            }
+        };
+        // eight sums a tile, one per product of a piece: short chains keep the error
+        // against 64 bits at the vector form's (1.1e-7 against 1.4e-7 relative at
+        // [6656, 19968]; a single sum doubled it)
+        f32x4 acc[RT][8];
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int s = 0; s < 8; ++s) acc[t][s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        const int sh = 16 * (c >> 1); // this lane's scale of a 64-quant pair of blocks
+        int m = wv;
+        if (m < np) load(m);
+        for (; m < np; m += NW) {
+            bf16x8 x[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) x[k] = ld_bf16x8(xp + 256 * int64_t(m) + 64 * (k / 2) + 8 * (k % 2));
+            Vec<uint32_t, 4> cw[RT][4], cd[RT];
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    *reinterpret_cast<Vec<uint32_t, 4> *>(lb + (16 * t + 4 * s + c) * PITCH + 16 * n) = w[t][s];
+                cd[t] = d[t];
+            }
+            if (m + NW < np) load(m + NW);
+            wave_lds_sync();
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    cw[t][s] = *reinterpret_cast<const Vec<uint32_t, 4> *>(lb + (16 * t + n) * PITCH + 64 * s + 16 * c);
+            wave_lds_sync();
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const float sc = f16_f32(uint16_t(cd[t].v[s] >> sh)), nsc = -128.0f * sc;
+                    uint32_t wb[8]; // bf16(q * d) in pairs, as above
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const uint32_t u = cw[t][s].v[k] ^ 0x80808080u;
+                        const float f0 = __builtin_fmaf(float(u & 0xffu), sc, nsc);
+                        const float f1 = __builtin_fmaf(float((u >> 8) & 0xffu), sc, nsc);
+                        const float f2 = __builtin_fmaf(float((u >> 16) & 0xffu), sc, nsc);
+                        const float f3 = __builtin_fmaf(float(u >> 24), sc, nsc);
+                        wb[2 * k] = uint32_t(__builtin_bit_cast(uint16_t, static_cast<__bf16>(f0))) |
+                                    (uint32_t(__builtin_bit_cast(uint16_t, static_cast<__bf16>(f1))) << 16);
+                        wb[2 * k + 1] = uint32_t(__builtin_bit_cast(uint16_t, static_cast<__bf16>(f2))) |
+                                        (uint32_t(__builtin_bit_cast(uint16_t, static_cast<__bf16>(f3))) << 16);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const Vec<uint32_t, 4> av{{wb[4 * i], wb[4 * i + 1], wb[4 * i + 2], wb[4 * i + 3]}};
+                        acc[t][2 * s + i] = mfma_bf16(__builtin_bit_cast(bf16x8, av), x[2 * s + i], acc[t][2 * s + i]);
+                    }
+                }
+        }
+#pragma unroll
+        for (int t = 0; t < RT; ++t) *reinterpret_cast<f32x4 *>(lb + 16 * (64 * t + lane)) = ((acc[t][0] + acc[t][1]) + (acc[t][2] + acc[t][3])) + ((acc[t][4] + acc[t][5]) + (acc[t][6] + acc[t][7]));
+        __syncthreads();
+        // lane (column n, c) holds weight rows 4c .. 4c + 3 of batch row n
+        for (int i = threadIdx.x; i < 256 * RT; i += 64 * NW) {
+            const int b = (i >> 4) & 15, t = i >> 8;
+            const int64_t o = r0 + 16 * t + (i & 15);
+            if (b >= B || o >= out) continue;
+            const int l = 16 * ((i & 15) >> 2) + b;
+            double s = 0.0;
+#pragma unroll
+            for (int k = 0; k < NW; ++k) s += *reinterpret_cast<const float *>(lw[k] + 16 * (64 * t + l) + 4 * (i & 3));
+            Y[b * ldy + o] = float(s);
+        }
+    }
+
     void launch_gemv_q8_0(mg_ctx *c, const int8_t *qs, const uint16_t *d, const uint16_t *x, int64_t batch,
                           int64_t rows, int64_t in, int64_t ldx, float *y, int64_t ldy, bool blockdot)
     {
@@ -285,6 +412,26 @@ namespace mg
         need(aligned16(qs) && aligned16(x) && ldx % 8 == 0, "gemv_q8_0: quants and activations must be 16-byte aligned");
         if (rows == 0) return;
         need(rows < (int64_t(1) << 33), "gemv_q8_0: too many rows");
+        // rows of whole 256-quant pieces: the matrix cores from two activation rows
+        // on (one row: 34-36 us against the vector form's 26 at [25600, 5120]); two
+        // rows only over a weight of 2^26 quants and more (10.4 us against 9.4 at
+        // [5120, 5120], 32-34 against 35 at [25600, 5120], 31 against 41 at [6656, 19968])
+        if ((batch > 2 || (batch == 2 && rows * in >= (int64_t(1) << 26))) && !blockdot && in % 256 == 0 && in > 0 && aligned16(d)) {
+            auto go = [&](auto kern, int64_t rt, int waves) {
+                hipLaunchKernelGGL(kern, dim3(unsigned((rows + 16 * rt - 1) / (16 * rt))), dim3(unsigned(64 * waves)), 0,
+                                   c->stream, qs, d, x, y, in, rows, ldx, ldy, int(batch));
+            };
+            // 16 rows and four waves a work-group, but 32 and eight where five or
+            // more activation rows weigh on fewer, longer weight rows (8 rows at
+            // [5120, 25600]: 41 us against 46; at [25600, 5120] 44 against 36, and
+            // under 4096 rows too few work-groups: 10.9 against 9.0 at [1024, 5120])
+            if (batch > 4 && rows >= 4096 && rows < 16384)
+                go(k_gemv_q8_0_mfma<2, 8>, 2, 8);
+            else
+                go(k_gemv_q8_0_mfma<1, 4>, 1, 4);
+            check_launch("k_gemv_q8_0_mfma");
+            return;
+        }
         const dim3 g{unsigned((rows + 3) / 4), 1u, 1u};
         // up to four activation rows per pass over the weights
         for (int64_t b0 = 0; b0 < batch; b0 += 4) {

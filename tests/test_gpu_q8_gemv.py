@@ -100,6 +100,40 @@ def test_gemv_widths(prims, n_in, blockdot):
     gemv_case(prims, 37, n_in, 1, blockdot, seed=61)
 
 
+@pytest.mark.parametrize("rows,n_in,B", ((1, 256, 2), (15, 512, 8), (17, 1280, 3), (33, 2304, 7), (4111, 256, 6),
+                                         (4127, 2304, 5), (16390, 512, 8)))
+def test_gemv_matrix_cores(prims, rows, n_in, B):
+    """two to eight activation rows over rows of whole 256-quant pieces: tiles of
+    16 and 32 weight rows with remainders, fewer pieces than waves, uneven pieces"""
+    gemv_case(prims, rows, n_in, B, False)
+
+
+def test_gemv_matrix_cores_strides_and_nonfinite(prims):
+    """strided activations and outputs; an infinite and a NaN activation row and
+    a weight row with an infinite scale reach only their own outputs"""
+    import torch
+    rows, n_in, B = 40, 512, 4
+    qs = torch.randint(-127, 128, (rows, n_in), dtype=torch.int8, device="cuda:0")
+    d = torch.full((rows, n_in // 32), 0.01, dtype=torch.float16, device="cuda:0")
+    d[7, 3] = float("inf")
+    x = torch.randn((B, n_in + 8), device="cuda:0").to(torch.bfloat16)
+    x[1, 5] = float("inf")
+    x[3, 6] = float("nan")
+    y = torch.full((B, rows + 3), 9.0, device="cuda:0")
+    prims.gemv_q8_0(qs, d, x[:, :n_in], y[:, :rows])
+    assert torch.all(y[:, rows:] == 9.0)
+    clean = [r for r in range(rows) if r != 7]
+    d16 = float(torch.tensor(0.01, dtype=torch.float16))
+    w = (qs.float() * d16).bfloat16().double()
+    ref = x[:, :n_in].double() @ w.t().contiguous()
+    bound = 1e-5 * (x[:, :n_in].double().abs() @ w.abs().t().contiguous())
+    for b in (0, 2):
+        assert torch.all((y[b, :rows].double() - ref[b]).abs()[clean] <= bound[b][clean])
+        assert not torch.isfinite(y[b, 7])
+    assert not torch.isfinite(y[1, :rows][qs[:, 5] != 0]).any()
+    assert torch.isnan(y[3, :rows]).all()
+
+
 def test_gemv_config5_shape(prims):
     """config 5's weight [25600, 5120] at decode (one token)"""
     gemv_case(prims, 25600, 5120, 1, False)
