@@ -32,8 +32,9 @@
 //                   (relative; bf16 carries 8 significant bits).
 // Online softmax per head in f32 (hardware exp2 on log2-scaled scores), the
 // running sums and O rows rescaled only in steps where a head's maximum
-// moved. Splits are at least 256 keys and long contexts get about one wave
-// per SIMD (1024 waves), each streaming its keys. A second kernel, one
+// moved. Splits are at least 64 keys up to 256 of them, then at least 256, and
+// long contexts get about one wave per SIMD (1024 waves), each streaming its
+// keys. A second kernel, one
 // work-group per (query head, 16 dims), merges the splits: global max, split
 // weights, the weighted sum of the split accumulators.
 #include "mg_device.hpp"
@@ -41,7 +42,9 @@
 
 namespace mg
 {
-    constexpr int kAttnSplit = 256;    // shortest split (keys)
+    constexpr int kAttnSplit = 256;    // shortest split (keys) past kAttnFine splits
+    constexpr int kAttnFineSplit = 64; // shortest split up to kAttnFine splits
+    constexpr int kAttnFine = 256;
     constexpr int kAttnWaves = 1024;   // splits x kv heads aimed at for long contexts
 
     struct AttnArgs
@@ -302,18 +305,35 @@ namespace mg
         need(total <= slots, "attn_decode: the attended keys do not fit the cache ring (qpos - lo + 1 > cache_slots)");
         // splits of at least 256 keys, few enough that a long context runs as
         // about one wave per SIMD, each streaming its keys with the next step's
-        // loads in flight; a multiple of 32 keys (one step)
-        int64_t ns = (total + kAttnSplit - 1) / kAttnSplit;
+        // loads in flight; a multiple of 32 keys (one step). Shorter contexts
+        // leave SIMDs idle and wait for one wave's chain of steps: up to 256
+        // splits they go down to 64 keys (32 q / 2 kv heads: 1500 keys 17.5 -> 9.6 us,
+        // 16000 18.3 -> 12.3, 32000 19.0 -> 15.3; 32-key splits 10.1, 15.1, 17.4, and
+        // more than 256 cost the combine more than they save, 65000 keys 20.9 ->
+        // 21.9), unless the workspace holds only the longer ones' partials.
         const int64_t ns_cap = kAttnWaves / (nkv * nsub) > 1 ? kAttnWaves / (nkv * nsub) : 1;
-        ns = ns < ns_cap ? ns : ns_cap;
-        int64_t per = (total + ns - 1) / ns;
-        per = (per + 31) / 32 * 32;
-        const int nsplit = int((total + per - 1) / per);
+        auto split = [&](int64_t ns, int64_t &per) {
+            ns = ns < ns_cap ? ns : ns_cap;
+            per = ((total + ns - 1) / ns + 31) / 32 * 32;
+            return (total + per - 1) / per;
+        };
+        auto partials = [&](int64_t n) { return ((2 * nq * n + 3) / 4 * 4 + nq * n * D) * int64_t(sizeof(float)); };
+        const int64_t ns = (total + kAttnSplit - 1) / kAttnSplit;
+        int64_t per, nsplit64 = split(ns, per);
+        if (ns < kAttnFine) {
+            const int64_t fine = (total + kAttnFineSplit - 1) / kAttnFineSplit;
+            int64_t fper;
+            const int64_t n = split(fine < kAttnFine ? fine : kAttnFine, fper);
+            if (partials(n) <= c->work_bytes) {
+                per = fper;
+                nsplit64 = n;
+            }
+        }
+        const int nsplit = int(nsplit64);
         // maxima and sums first, then the partial outputs from a 16-byte boundary
         // (the combine reads them as 16-byte vectors)
         const int64_t pa_off = (2 * nq * nsplit + 3) / 4 * 4;
-        const int64_t need_bytes = (pa_off + nq * nsplit * D) * int64_t(sizeof(float));
-        need(need_bytes <= c->work_bytes, "attn_decode: partials exceed the context workspace (raise workspace_bytes at mg_open)");
+        need(partials(nsplit) <= c->work_bytes, "attn_decode: partials exceed the context workspace (raise workspace_bytes at mg_open)");
         float *pm = static_cast<float *>(c->work);
         float *pl = pm + nq * nsplit;
         float *pa = pm + pa_off;

@@ -107,3 +107,19 @@ def test_errors(prims):
     q = torch.zeros((8, 128), dtype=torch.bfloat16, device="cuda:0")
     with pytest.raises(Exception, match="cache ring"):
         prims.attn_decode(q, kc, kc, 100, 0.1)
+
+
+@pytest.mark.parametrize("nq,nkv,keys", ((32, 2, 1), (32, 2, 63), (32, 2, 65), (40, 8, 129), (32, 2, 1500), (8, 1, 16385),
+                                         (40, 8, 8193)))
+def test_short_splits(prims, nq, nkv, keys):
+    """contexts of at most 256 splits run in 64-key ones: one key, a split's edges,
+    a last split of one key, the step from 64 to longer splits"""
+    attn_case(prims, nq, nkv, 128, keys + 7, keys - 1, seed=97)
+
+
+def test_small_workspace_takes_the_longer_splits(prims):
+    """a workspace that holds the partials of 256-key splits only"""
+    import mgprims
+    small = mgprims.Prims(0, workspace_bytes=8 * 8 * (2 + 128) * 4)
+    attn_case(small, 8, 2, 128, 2048, 2047, seed=98)
+    small.close()
