@@ -192,7 +192,6 @@ namespace mg
     // work-group reduction scratch, and each kernel's LDS around it
     struct SfRed
     {
-        double red[kSfThreads];
         double redd[kSfThreads / 64];
         uint64_t redu[kSfThreads / 64];
         uint32_t bc[4];     // broadcast words
@@ -264,23 +263,17 @@ namespace mg
         *tot = all;
         return base + incl - v;
     }
-    // the same for f64 values: each thread's exclusive prefix, summed in a
-    // fixed order (the lanes' values through LDS, then the waves')
+    // the same for f64 values: each thread's exclusive prefix, in a fixed order
+    // (lanes by doubling steps, then the waves' totals in order)
     MG_DEV double sf_scan_f64(double v, SfRed &L)
     {
-        L.red[threadIdx.x] = v;
-        __syncthreads();
-        const int w0 = int(threadIdx.x) & ~63, lane = int(threadIdx.x) & 63;
-        double in_wave = 0.0;
-        for (int i = 0; i < lane; ++i) in_wave += L.red[w0 + i];
-        double wave_tot = in_wave;
-        for (int i = lane; i < 64; ++i) wave_tot += L.red[w0 + i];
-        if (lane == 63) L.redd[threadIdx.x >> 6] = wave_tot;
+        const double incl = wave_incl_scan(v);
+        if ((threadIdx.x & 63) == 63) L.redd[threadIdx.x >> 6] = incl;
         __syncthreads();
         double base = 0.0;
         for (int i = 0; i < int(threadIdx.x >> 6); ++i) base += L.redd[i];
         __syncthreads();
-        return base + in_wave;
+        return base + (incl - v);
     }
 
     // keys[0, n) sorted descending, n a power of two: each wave sorts its n/16
@@ -525,8 +518,9 @@ namespace mg
     // desc, index asc) order (ncand = |C|, S its e sum, mx its maximum): the
     // top_p and min_p cuts as prefixes of that order, then softmax(x / T)
     // over the kept prefix into oi / op and its length into *out_n (-1 when
-    // the cut lies past the ng keys at hand).
-    MG_DEV void sf_emit_sorted(SfRed &L, const uint64_t *keys, int64_t ng, int64_t ncand, double S, float mx,
+    // the cut lies past kSortMax keys); false, nothing written, when it lies past
+    // the ng < kSortMax keys at hand.
+    MG_DEV bool sf_emit_sorted(SfRed &L, const uint64_t *keys, int64_t ng, int64_t ncand, double S, float mx,
                                float temperature, float top_p, float min_p, int64_t *oi, float *op, int64_t *out_n)
     {
         const float pmax = float(1.0 / S), thr = min_p * pmax;
@@ -571,21 +565,25 @@ namespace mg
             n = nmt < n ? nmt : n;
         }
         if (n > ng) {
+            if (ng < kSortMax) return false;
             if (threadIdx.x == 0) *out_n = -1;
-            return;
+            return true;
         }
         double F = 0.0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (t0 + e < n) F += double(exp_diff(xv[e] / temperature, y0));
+        for (int e = 0; e < 4; ++e) {
+            ev[e] = t0 + e < n ? double(exp_diff(xv[e] / temperature, y0)) : 0.0;
+            F += ev[e];
+        }
         F = sf_sum_f64(F, L);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (t0 + e < n) {
                 oi[t0 + e] = int64_t(0xffffffffu - uint32_t(keys[t0 + e]));
-                op[t0 + e] = float(double(exp_diff(xv[e] / temperature, y0)) / F);
+                op[t0 + e] = float(ev[e] / F);
             }
         if (threadIdx.x == 0) *out_n = n;
+        return true;
     }
 
     // region 0 (keys[0, n0)) sorted; region 1 (keys[kSortMax, kSortMax + n1)),
@@ -804,9 +802,9 @@ namespace mg
     }
 
     // ------------------------------------------------ split rows (sorted, no top_k cut)
-    // Rows with sorted outputs and every candidate in C (top_k <= 0 or >= V)
-    // split over G work-groups per row, one slice of slen entries each (64
-    // rows then fill the chip): pass 1 per slice with its prefix histogram
+    // 65 to 128 rows (fewer take the register slices below) with sorted outputs
+    // and every candidate in C (top_k <= 0 or >= V), split over G work-groups per
+    // row, one slice of slen entries each: pass 1 per slice with its prefix histogram
     // (k_sample_split_stats), the row's decision from the slices' counts
     // (k_sample_split_decide: the point masses, the threshold bin bstar, and
     // where each slice's keys go), S per slice with the gathering into the
@@ -1162,6 +1160,359 @@ namespace mg
                        out_p + row * V, out_n + row);
     }
 
+    // ------------------------------------------- register slices (up to 64 rows)
+    // The same rows, up to 64 of them, over G = 16 or 8 work-groups each. A slice is every G-th KiB of the row (a
+    // language model's frequent tokens sit side by side: neighbours fall to
+    // different slices), held in its work-group's registers, so the logits are
+    // read once:
+    //   k_sample_slice   the slice's maximum, counts and S relative to that
+    //                    maximum; its largest keys, at most M = 8192 / G of them,
+    //                    sorted: those from T0 up, a rank among the threads' maxima
+    //                    (0.8 M keys of a random row), or, where more than M reach
+    //                    T0, those in the image-prefix bins that hold at most M;
+    //   k_sample_finish  per row: S = sum S_g e^(m_g - m) (f64 exponentials), the
+    //                    slices' runs merged two by two, the cut and the outputs.
+    // Every slice also gives L, an image from which up its run is complete. Above
+    // the largest L the merged keys are the row's largest in order, so a cut found
+    // there, or more than kSortMax keys kept there, is exact. Rows whose cut lies
+    // deeper (a bin of more than M equal or near-equal values above the cut, one
+    // slice holding much more of the row's head than the others) run the
+    // one-work-group algorithm (sample_row) in the finishing work-group with the
+    // same S: the same selection and the same bits.
+    // The two kernels are bound by their chains of reductions, the sort of a run
+    // and the merges, not by the logits: top_p 0.95, rows of 201088, 1 row 86 -> 51
+    // us, 8 rows 89 -> 50, 32 rows 91 -> 62, 64 rows 86 -> 85 against the four kernels
+    // above, which stay ahead past 64 (100 rows: 100 against 126).
+    constexpr int kSliceKeys = 2 * kSortMax; // keys of a row's runs together
+    constexpr int kSliceMax = 16;            // slices per row
+    constexpr int kSliceVec = 7;             // 16-byte vectors a thread holds at most
+
+    struct SliceStat
+    {
+        double S;       // sum of e^(x - m) over the slice's candidates
+        uint64_t best;  // (image with NaN on top) << 32 | ~index, where a point mass may need it
+        uint32_t mk;    // image of the candidates' maximum (0: none)
+        uint32_t nc;    // candidates
+        uint32_t nfin;  // finite entries
+        uint32_t nrun;  // keys in the run
+        uint32_t from;  // the run holds every key with an image >= from
+        uint32_t pad;
+    };
+    struct SliceWork
+    {
+        SliceStat *stat; // [rows][G]
+        uint64_t *keys;  // [rows][G][M]
+        int M;
+    };
+    struct SfSliceLds : SfRed
+    {
+        uint32_t hist[1 << kHistBits];
+        uint64_t keys[kSliceKeys / 8];
+        uint32_t count;
+    };
+    struct SfRunsLds : SfRed
+    {
+        uint64_t keys[2][kSliceKeys];
+        int len[kSliceMax];
+    };
+
+    // kRank: for NV * 4 random entries a thread, about 0.8 M keys lie at or above the
+    // kRank-th largest of 64 thread maxima (M = 1024 at NV 7, 512 at NV 4)
+    template <int NV, int kRank>
+    __global__ __launch_bounds__(kSfThreads) void k_sample_slice(const float *__restrict__ lg, int64_t ld, int64_t V,
+                                                                float temperature, SliceWork w)
+    {
+        __shared__ SfSliceLds L;
+        constexpr int kBins = 1 << kHistBits, BPT = kBins / kSfThreads;
+        const int G = int(gridDim.x), g = int(blockIdx.x);
+        const int64_t row = blockIdx.y;
+        const int wv = int(threadIdx.x >> 6), lane = int(threadIdx.x & 63);
+        // thread's vector i: the KiB (16 i + wave) G + g of the row, entries past V
+        // read as -inf (out of the buffer's range); a row aligned to its floats
+        const auto rs = buf_rsrc(lg + row * ld, int(V) * 4);
+        float x[NV][4];
+        auto first = [&](int i) { return (((i * 16 + wv) * G + g) * 64 + lane) * 4; };
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const Vec<float, 4> v = buf_ld16<float, 4, 0>(rs, first(i) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[i][e] = v.v[e];
+        }
+        // the thread's maximum (NaN dropped) and counts
+        float m1 = -__builtin_huge_valf();
+        uint32_t nc = 0, nfin = 0;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                x[i][e] = first(i) + e < int(V) ? x[i][e] : -__builtin_huge_valf();
+                m1 = __builtin_fmaxf(m1, x[i][e]);
+                nc += sf_cand(x[i][e]) ? 1u : 0u;
+                nfin += __builtin_isfinite(x[i][e]) ? 1u : 0u;
+            }
+        // the slice's counts and maximum, and T0: each wave's kRank-th largest thread
+        // maximum, the eighth largest of those over the waves
+        const uint64_t cnt = sf_sum_u64((uint64_t(nc) << 32) | nfin, L);
+        nc = uint32_t(cnt >> 32);
+        nfin = uint32_t(cnt);
+        uint32_t im[1] = {f32_key(m1 + 0.0f)};
+        wave_bitonic_desc<uint32_t, 1>(im);
+        if (lane == 0) L.redu[wv] = (uint64_t(im[0]) << 32) | uint32_t(__builtin_amdgcn_readlane(int(im[0]), kRank - 1));
+        __syncthreads();
+        const uint64_t wm = L.redu[lane & 15];
+        const uint32_t big = dpp_max_u32(uint32_t(wm >> 32)), mid = uint32_t(wm);
+        int above = 0;
+#pragma unroll
+        for (int i = 0; i < kSfThreads / 64; ++i) {
+            const uint32_t o = uint32_t(__builtin_amdgcn_readlane(int(mid), i));
+            above += o > mid || (o == mid && i < (lane & 15)) ? 1 : 0;
+        }
+        const uint32_t t0 = uint32_t(__builtin_amdgcn_readlane(int(mid), int(__builtin_ctzll(__builtin_amdgcn_ballot_w64(above == 7)))));
+        const float mx = key_f32(big);
+        float T0 = key_f32(t0);
+        __syncthreads();
+        SliceStat st{};
+        st.nc = nc;
+        st.nfin = nfin;
+        st.mk = nc ? big : 0u;
+        if (nfin == 0 || !(temperature > 0.0f)) {
+            // a point mass may take np.argmax: the first largest, NaN on top
+            uint64_t best = 0;
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t hi = x[i][e] != x[i][e] ? 0xffffffffu : sf_img(x[i][e]);
+                    const uint64_t k = (uint64_t(hi) << 32) | uint64_t(0xffffffffu - uint32_t(first(i) + e));
+                    best = first(i) + e < int(V) && k > best ? k : best;
+                }
+            st.best = sf_max_u64(best, L);
+        }
+        // a slice of no use to the order: no candidates, or +inf (the row's count is -1)
+        if (nc == 0 || !(mx < __builtin_huge_valf()) || !(temperature > 0.0f)) {
+            if (threadIdx.x == 0) w.stat[row * G + g] = st;
+            return;
+        }
+        double S = 0.0;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S += sf_cand(x[i][e]) ? double(exp_diff(x[i][e], mx)) : 0.0;
+        st.S = sf_sum_f64(S, L);
+        // the keys from T0 up: the run, when M hold them
+        uint32_t top = 0;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) top += sf_cand(x[i][e]) && x[i][e] >= T0 ? 1u : 0u;
+        int tot;
+        int at = sf_scan(int(top), L, &tot);
+        uint32_t from = uint32_t(tot) == nc ? 0u : t0;
+        const bool binned = tot > w.M; // (uniform)
+        if (binned) {
+#pragma unroll
+            for (int b = 0; b < BPT; ++b) L.hist[b * kSfThreads + int(threadIdx.x)] = 0;
+            if (threadIdx.x == 0) {
+                L.count = 0;
+                L.bc[0] = 0;
+            }
+            __syncthreads();
+            __asm__ volatile("" : "+v"(T0));
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (sf_cand(x[i][e]) && x[i][e] >= T0) atomicAdd(&L.hist[sf_img(x[i][e]) >> (32 - kHistBits)], 1u);
+            __syncthreads();
+            // thread t holds bins kBins-1-BPT*t-e: its exclusive prefix counts the
+            // keys in higher bins; the first bin that passes M ends the run
+            uint32_t c[BPT];
+            int own = 0;
+#pragma unroll
+            for (int e = 0; e < BPT; ++e) {
+                c[e] = L.hist[kBins - 1 - BPT * int(threadIdx.x) - e];
+                own += int(c[e]);
+            }
+            int all;
+            int acc = sf_scan(own, L, &all);
+#pragma unroll
+            for (int e = 0; e < BPT; ++e) {
+                if (acc <= w.M && acc + int(c[e]) > w.M) L.bc[0] = uint32_t(kBins - 1 - BPT * int(threadIdx.x) - e) + 1u;
+                acc += int(c[e]);
+            }
+            __syncthreads();
+            from = L.bc[0] >= uint32_t(kBins) ? 0xffffffffu : L.bc[0] << (32 - kHistBits);
+        }
+        st.from = from;
+        __asm__ volatile("" : "+v"(T0)); // compares afresh: 4 NV kept masks would spill
+        // at most M keys, in any order (unique, sorted next): a thread's from its
+        // place in the scan, or, where the bins cut among them, from a counter
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (sf_cand(x[i][e]) && x[i][e] >= T0) {
+                    const uint32_t img = sf_img(x[i][e]);
+                    const uint64_t key = (uint64_t(img) << 32) | uint64_t(0xffffffffu - uint32_t(first(i) + e));
+                    if (!binned)
+                        L.keys[at++] = key;
+                    else if (img >= from)
+                        L.keys[atomicAdd(&L.count, 1u)] = key;
+                }
+        __syncthreads();
+        const int n = binned ? int(L.count) : tot; // at most M <= 1024
+        if (n + int(threadIdx.x) < kSfThreads) L.keys[n + int(threadIdx.x)] = 0; // zeros sort last
+        __syncthreads();
+        sf_sort_regs<1>(L.keys, kSfThreads);
+        uint64_t *out = w.keys + (row * G + g) * int64_t(w.M);
+        for (int i = threadIdx.x; i < n; i += kSfThreads) out[i] = L.keys[i];
+        st.nrun = uint32_t(n);
+        if (threadIdx.x == 0) w.stat[row * G + g] = st;
+    }
+
+    // how many of the descending keys[0, n) are larger than k
+    MG_DEV int sf_larger(const uint64_t *keys, int n, uint64_t k)
+    {
+        int a = 0, b = n;
+        while (a < b) {
+            const int m = (a + b) >> 1;
+            if (keys[m] > k)
+                a = m + 1;
+            else
+                b = m;
+        }
+        return a;
+    }
+
+    __global__ __launch_bounds__(kSfThreads) void k_sample_finish(const float *__restrict__ lg, int64_t ld, int64_t V,
+                                                                 const int64_t *__restrict__ raw_amax, int64_t top_k,
+                                                                 int G, float temperature, float top_p, float min_p,
+                                                                 int64_t *__restrict__ out_ids,
+                                                                 float *__restrict__ out_p,
+                                                                 int64_t *__restrict__ out_n, SliceWork w)
+    {
+        __shared__ union
+        {
+            SfRunsLds m;
+            SfLds full;
+        } U;
+        SfRunsLds &L = U.m;
+        const int64_t row = blockIdx.x;
+        // the runs as they lie in memory (run r from r M) and the slices' numbers,
+        // one a lane, all requested together
+        const int M = w.M, lane = int(threadIdx.x & 63);
+        const uint64_t *src = w.keys + row * int64_t(kSliceKeys);
+        constexpr int KPT = kSliceKeys / kSfThreads;
+        uint64_t kv[KPT];
+#pragma unroll
+        for (int k = 0; k < KPT; ++k) kv[k] = src[k * kSfThreads + int(threadIdx.x)];
+        SliceStat my = w.stat[row * G + (lane < G ? lane : 0)];
+        if (lane >= G) my.nc = my.nfin = my.mk = my.nrun = my.from = 0;
+        const uint64_t nfin = wave_sum(uint64_t(my.nfin)), nc = wave_sum(uint64_t(my.nc));
+        const uint64_t best = wave_max(my.best); // (lanes past G repeat the first's)
+        const uint32_t mk = dpp_max_u32(my.mk), from = dpp_max_u32(my.nc ? my.from : 0u);
+        int64_t *oi = out_ids + row * V;
+        float *op = out_p + row * V;
+        if (nfin == 0 || !(temperature > 0.0f)) {
+            if (threadIdx.x == 0) {
+                oi[0] = nfin == 0 && raw_amax ? raw_amax[row] : int64_t(0xffffffffu - uint32_t(best));
+                op[0] = 1.0f;
+                out_n[row] = 1;
+            }
+            return;
+        }
+        const float mx = key_f32(mk);
+        if (!(mx < __builtin_huge_valf())) { // +inf among the candidates
+            if (threadIdx.x == 0) out_n[row] = -1;
+            return;
+        }
+        const double S = dpp_sum(my.nc ? my.S * (my.mk == mk ? 1.0 : mgm::exp(double(key_f32(my.mk)) - double(mx))) : 0.0);
+        // slots past a run's end hold nothing: 0, below every key
+        if (threadIdx.x < kSliceMax) L.len[threadIdx.x] = int(my.nc ? my.nrun : 0u);
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < KPT; ++k) {
+            const int i = k * kSfThreads + int(threadIdx.x);
+            kv[k] = i % M < L.len[i / M] ? kv[k] : 0;
+            L.keys[0][i] = kv[k];
+        }
+        // The keys past the top_p cut need no merging: the e of 64 keys in a row goes
+        // to the prefix bin of the smallest (f32 sums in any order: a margin of 2^-10
+        // covers them), and the bin where they pass top_p S ends the runs: a little
+        // past the cut, never ahead of it. The exact cut comes after.
+        uint32_t floor_ = 0;
+        if (top_p < 1.0f) {
+            constexpr int kBins = 1 << kHistBits, BPT = kBins / kSfThreads;
+            float *wt = reinterpret_cast<float *>(L.keys[1]);
+#pragma unroll
+            for (int b = 0; b < BPT; ++b) wt[b * kSfThreads + int(threadIdx.x)] = 0.0f;
+            if (threadIdx.x == 0) L.bc[0] = 0;
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < KPT; ++k) {
+                const uint32_t img = uint32_t(kv[k] >> 32);
+                const float e = dpp_sum_f32(img ? __builtin_amdgcn_exp2f((key_f32(img) - mx) * 1.44269504f) : 0.0f);
+                const uint32_t last = dpp_min_u32(img ? img : 0xffffffffu);
+                if (lane == 0 && last != 0xffffffffu) atomicAdd(&wt[last >> (32 - kHistBits)], e);
+            }
+            __syncthreads();
+            double c[BPT], own = 0.0;
+#pragma unroll
+            for (int e = 0; e < BPT; ++e) {
+                c[e] = double(wt[kBins - 1 - BPT * int(threadIdx.x) - e]);
+                own += c[e];
+            }
+            double acc = sf_scan_f64(own, L);
+            const double target = double(top_p) * S * (1.0 + 0x1p-10);
+#pragma unroll
+            for (int e = 0; e < BPT; ++e) {
+                if (acc < target && acc + c[e] >= target) L.bc[0] = uint32_t(kBins - 1 - BPT * int(threadIdx.x) - e);
+                acc += c[e];
+            }
+            __syncthreads();
+            floor_ = L.bc[0] << (32 - kHistBits); // 0: the cut lies past the keys at hand
+        }
+        const uint32_t low = floor_ > from ? floor_ : from;
+        __syncthreads(); // (the runs are in LDS where no sums were taken)
+        if (int(threadIdx.x) < G) {
+            // keys >= low: a prefix (0xffffffff in `from`: none)
+            const uint64_t lowest = uint64_t(low) << 32;
+            const int n = L.len[threadIdx.x];
+            L.len[threadIdx.x] = from == 0xffffffffu ? 0 : sf_larger(L.keys[0] + int(threadIdx.x) * M, n, lowest ? lowest - 1 : 0);
+        }
+        __syncthreads();
+        // merged two by two, run r of a level from r * size: each key to its index
+        // in its run plus the larger keys of the other (the keys are unique), the
+        // first kSortMax of every merged run kept
+        int cur = 0;
+        for (int runs = G, size = M; runs > 1; runs >>= 1, size *= 2) {
+            const uint64_t *from_ = L.keys[cur];
+            uint64_t *to = L.keys[cur ^ 1];
+#pragma unroll
+            for (int k = 0; k < KPT; ++k) {
+                const int i = k * kSfThreads + int(threadIdx.x);
+                const int r = i / size, at = i % size;
+                if (at < L.len[r]) {
+                    const uint64_t key = from_[i];
+                    const int pos = at + sf_larger(from_ + (r ^ 1) * size, L.len[r ^ 1], key);
+                    if (pos < kSortMax) to[(r >> 1) * 2 * size + pos] = key;
+                }
+            }
+            __syncthreads();
+            int n = 0;
+            if (int(threadIdx.x) < runs / 2) n = L.len[2 * threadIdx.x] + L.len[2 * threadIdx.x + 1];
+            __syncthreads();
+            if (int(threadIdx.x) < runs / 2) L.len[threadIdx.x] = n < kSortMax ? n : kSortMax;
+            __syncthreads();
+            cur ^= 1;
+        }
+        const int64_t ng = L.len[0];
+        if (sf_emit_sorted(L, L.keys[cur], ng, int64_t(nc), S, mx, temperature, top_p, min_p, oi, op, out_n + row))
+            return;
+        __syncthreads();
+        sample_row(U.full, row, lg, ld, V, raw_amax, top_k, temperature, top_p, min_p, out_ids, out_p, out_n, S);
+    }
+
     void launch_sample_rows(mg_ctx *c, const float *lg, int64_t ld, int64_t rows, int64_t V,
                             const int64_t *raw_amax, int64_t top_k, double temperature, double top_p, double min_p,
                             int64_t *out_ids, float *out_p, int64_t *out_n)
@@ -1173,9 +1524,36 @@ namespace mg
         need(ld >= V, "sample_rows: row stride < V");
         if (rows == 0) return;
         const float T = float(temperature), tp = float(top_p), mp = float(min_p);
-        // the split path: sorted outputs with no top_k cut, few enough rows that
-        // G >= 2 work-groups per row fill the chip, and room in the workspace
+        // sorted outputs with no top_k cut, up to 64 rows: slices that fit the
+        // registers and runs that fit the workspace; 16 slices a row up to 16 rows,
+        // else 8, and 16 where 8 do not hold V
         const bool sorted = top_k > 0 || tp < 1.0f;
+        auto vecs = [&](int G) { return ((V + 3) / 4 + int64_t(kSfThreads) * G - 1) / (int64_t(kSfThreads) * G); };
+        int GS = rows <= 16 ? 16 : 8;
+        while (GS < kSliceMax && vecs(GS) > kSliceVec) GS *= 2;
+        const int64_t b_slice = (rows * GS * int64_t(sizeof(SliceStat)) + 255) / 256 * 256;
+        if (sorted && (top_k <= 0 || top_k >= V) && rows <= 64 && V >= 4 * 4096 && vecs(GS) <= kSliceVec &&
+            b_slice + rows * kSliceKeys * 8 <= c->work_bytes) {
+            SliceWork sw;
+            sw.stat = static_cast<SliceStat *>(c->work);
+            sw.keys = reinterpret_cast<uint64_t *>(static_cast<char *>(c->work) + b_slice);
+            sw.M = kSliceKeys / GS;
+            auto go = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(unsigned(GS), unsigned(rows)), dim3(kSfThreads), 0, c->stream, lg, ld, V, T, sw);
+            };
+            const int64_t nv = vecs(GS);
+            if (nv <= 4)
+                go(k_sample_slice<4, 21>);
+            else
+                go(k_sample_slice<kSliceVec, 35>);
+            check_launch("k_sample_slice");
+            hipLaunchKernelGGL(k_sample_finish, dim3(unsigned(rows)), dim3(kSfThreads), 0, c->stream, lg, ld, V,
+                               raw_amax, top_k, GS, T, tp, mp, out_ids, out_p, out_n, sw);
+            check_launch("k_sample_finish");
+            return;
+        }
+        // the split path: the same rows where those do not apply, few enough that
+        // G >= 2 work-groups per row fill the chip, and room in the workspace
         const int G = int(rows <= 256 / kSplitMax ? kSplitMax : 256 / rows);
         constexpr int64_t kBins = int64_t(1) << kHistBits;
         auto al = [](int64_t b) { return (b + 255) / 256 * 256; };

@@ -365,6 +365,47 @@ def test_sample_rows_split_random(prims, case):
         assert np.abs(probs[r, :n[r]].astype(np.float64) - wp).max() <= 2e-6, (case, r)
 
 
+@pytest.mark.parametrize("rows,V,sigma", ((2, 201088, 3.0), (17, 201088, 2.5), (3, 16384, 3.0), (5, 16387, 2.5),
+                                          (40, 65536, 3.0)))
+def test_sample_rows_uneven_slices(prims, rows, V, sigma):
+    """the head of the order in one register slice only (every 16th or 8th KiB of
+    the row raised), so its run does not reach the cut and the row is finished by
+    the one-work-group algorithm; beside it rows of equal values past M in every
+    slice under a short nucleus, and rows of one candidate"""
+    import torch
+    rng = np.random.default_rng(60 + rows)
+    G = 16 if rows <= 16 else 8
+    L = (rng.standard_normal((rows, V)) * sigma).astype(np.float32)
+    L[0, (np.arange(V) // 256) % G == 3] += np.float32(30.0)
+    L[1] = np.float32(1.0)
+    L[1, rng.permutation(V)[:50]] = rng.uniform(30.0, 33.0, 50).astype(np.float32)
+    if rows > 2:
+        L[2] = -np.inf
+        L[2, V - 1] = 2.0
+    keep = []
+    for r in range(rows):
+        x = np.sort(L[r][np.isfinite(L[r])])[::-1]
+        e32 = np.exp(x - x[0])
+        p64 = softmax(x.astype(np.float64))
+        c32 = np.searchsorted(np.cumsum(e32 / e32.sum()), np.float32(0.9)) + 1
+        c64 = np.searchsorted(np.cumsum(p64), np.float64(np.float32(0.9))) + 1
+        keep.append(c32 == c64 or min(c32, c64) > 4096)
+    assert keep[1] and sum(keep) >= rows - 2
+    want = O.sample_rows(L, np.argmax(L, axis=1), 0, 1.0, 0.9, 0.0)
+    ids, probs, n = prims.sample_rows(torch.from_numpy(L).cuda(), 0, 1.0, 0.9, 0.0)
+    ids, probs, n = ids.cpu().numpy(), probs.cpu().numpy(), n.cpu().numpy()
+    for r in range(rows):
+        if not keep[r]:
+            continue
+        wi, wp = want[r]
+        if len(wi) > 4096:
+            assert n[r] == -1, r
+            continue
+        assert n[r] == len(wi), (r, n[r], len(wi))
+        assert np.array_equal(ids[r, :n[r]], wi), r
+        assert np.abs(probs[r, :n[r]].astype(np.float64) - wp).max() <= 2e-6, r
+
+
 def test_sample_rows_left_to_host(prims):
     """count -1: a nucleus of more than 4096 sorted candidates (flat logits), and a
     row holding +inf (the reference's probabilities are NaN there); other rows of
