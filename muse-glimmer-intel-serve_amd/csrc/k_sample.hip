@@ -1180,9 +1180,11 @@ namespace mg
     // one-work-group algorithm (sample_row) in the finishing work-group with the
     // same S: the same selection and the same bits.
     // The two kernels are bound by their chains of reductions, the sort of a run
-    // and the merges, not by the logits: top_p 0.95, rows of 201088, 1 row 86 -> 51
-    // us, 8 rows 89 -> 50, 32 rows 91 -> 62, 64 rows 86 -> 85 against the four kernels
-    // above, which stay ahead past 64 (100 rows: 100 against 126).
+    // and the merges, not by the logits. Slice + finish in the trace, top_p 0.95, rows
+    // of 201088: 1 row 15.6 + 24.5 us, 8 rows 16.4 + 25.2, 32 rows 25.2 + 25.3, 64 rows
+    // 50.2 + 25.5 (a work-group's registers fill a CU: two rounds; held to half of them
+    // the slices spill, 85.8). The four kernels above take 86 to 91 us for any of these;
+    // past 64 rows they stay ahead (100 rows: 100 us against about 114).
     constexpr int kSliceKeys = 2 * kSortMax; // keys of a row's runs together
     constexpr int kSliceMax = 16;            // slices per row
     constexpr int kSliceVec = 7;             // 16-byte vectors a thread holds at most
@@ -1213,7 +1215,7 @@ namespace mg
     struct SfRunsLds : SfRed
     {
         uint64_t keys[2][kSliceKeys];
-        int len[kSliceMax];
+        int len[2][kSliceMax];
     };
 
     // kRank: for NV * 4 random entries a thread, about 0.8 M keys lie at or above the
@@ -1370,20 +1372,6 @@ namespace mg
         if (threadIdx.x == 0) w.stat[row * G + g] = st;
     }
 
-    // how many of the descending keys[0, n) are larger than k
-    MG_DEV int sf_larger(const uint64_t *keys, int n, uint64_t k)
-    {
-        int a = 0, b = n;
-        while (a < b) {
-            const int m = (a + b) >> 1;
-            if (keys[m] > k)
-                a = m + 1;
-            else
-                b = m;
-        }
-        return a;
-    }
-
     __global__ __launch_bounds__(kSfThreads) void k_sample_finish(const float *__restrict__ lg, int64_t ld, int64_t V,
                                                                  const int64_t *__restrict__ raw_amax, int64_t top_k,
                                                                  int G, float temperature, float top_p, float min_p,
@@ -1427,15 +1415,17 @@ namespace mg
             return;
         }
         const double S = dpp_sum(my.nc ? my.S * (my.mk == mk ? 1.0 : mgm::exp(double(key_f32(my.mk)) - double(mx))) : 0.0);
-        // slots past a run's end hold nothing: 0, below every key
-        if (threadIdx.x < kSliceMax) L.len[threadIdx.x] = int(my.nc ? my.nrun : 0u);
-        __syncthreads();
+        // slots past a run's end hold nothing: 0, below every key (a wave's 64 lie in one run)
+        const int lm = 31 - __builtin_clz(unsigned(M));
+        const int nrun = int(my.nc ? my.nrun : 0u);
+        const int wave0 = __builtin_amdgcn_readfirstlane(int(threadIdx.x) & ~63);
 #pragma unroll
         for (int k = 0; k < KPT; ++k) {
-            const int i = k * kSfThreads + int(threadIdx.x);
-            kv[k] = i % M < L.len[i / M] ? kv[k] : 0;
-            L.keys[0][i] = kv[k];
+            const int i = k * kSfThreads + wave0;
+            kv[k] = (i & (M - 1)) + lane < __builtin_amdgcn_readlane(nrun, i >> lm) ? kv[k] : 0;
         }
+        if (threadIdx.x < kSliceMax) L.len[0][threadIdx.x] = 0;
+        __syncthreads();
         // The keys past the top_p cut need no merging: the e of 64 keys in a row goes
         // to the prefix bin of the smallest (f32 sums in any order: a margin of 2^-10
         // covers them), and the bin where they pass top_p S ends the runs: a little
@@ -1472,41 +1462,91 @@ namespace mg
             __syncthreads();
             floor_ = L.bc[0] << (32 - kHistBits); // 0: the cut lies past the keys at hand
         }
+        // the runs' keys from low up (a prefix of each; none where `from` says so), one
+        // run after the other in LDS
         const uint32_t low = floor_ > from ? floor_ : from;
-        __syncthreads(); // (the runs are in LDS where no sums were taken)
-        if (int(threadIdx.x) < G) {
-            // keys >= low: a prefix (0xffffffff in `from`: none)
-            const uint64_t lowest = uint64_t(low) << 32;
-            const int n = L.len[threadIdx.x];
-            L.len[threadIdx.x] = from == 0xffffffffu ? 0 : sf_larger(L.keys[0] + int(threadIdx.x) * M, n, lowest ? lowest - 1 : 0);
+        bool in[KPT];
+#pragma unroll
+        for (int k = 0; k < KPT; ++k) {
+            in[k] = kv[k] != 0 && uint32_t(kv[k] >> 32) >= low && from != 0xffffffffu;
+            const int n = __builtin_popcountll(__builtin_amdgcn_ballot_w64(in[k]));
+            if (lane == 0 && n) atomicAdd(&L.len[0][(k * kSfThreads + wave0) >> lm], n);
+        }
+        __syncthreads(); // (the bins' sums in keys[1] are read)
+        const int rl = lane < G ? L.len[0][lane] : 0, upto = wave_prefix_sum(rl);
+        int cur = 0, total = __builtin_amdgcn_readlane(upto, 63);
+#pragma unroll
+        for (int k = 0; k < KPT; ++k) {
+            const int i = k * kSfThreads + wave0;
+            const int at = __builtin_amdgcn_readlane(upto - rl, i >> lm) + (i & (M - 1)) + lane;
+            if (in[k]) L.keys[0][at] = kv[k];
         }
         __syncthreads();
-        // merged two by two, run r of a level from r * size: each key to its index
-        // in its run plus the larger keys of the other (the keys are unique), the
-        // first kSortMax of every merged run kept
-        int cur = 0;
-        for (int runs = G, size = M; runs > 1; runs >>= 1, size *= 2) {
+        // merged two by two, the first kSortMax keys of every merged run kept. A
+        // thread writes four keys in a row: one bisection finds how many of the keys
+        // ahead of them either run gives (the keys are unique), then they are taken
+        // in order. (One bisection a key was bound by its instructions, 5 us a level for
+        // 3300 keys: the kernel 37.4 us at 1 row, 37.5 at 64, now 24.5 and 25.5.)
+        constexpr int KO = 4; // keys a thread writes in a row
+        for (int runs = G; runs > 1; runs >>= 1) {
             const uint64_t *from_ = L.keys[cur];
             uint64_t *to = L.keys[cur ^ 1];
+            const int *len = L.len[cur];
+            for (int c0 = 0;; c0 += kSfThreads) {
+                // the pair of runs this thread's keys come from
+                const int c = c0 + int(threadIdx.x);
+                int base = 0, out = 0, chunks = 0;
+                int pa = 0, na = 0, nb = 0, n = 0, po = 0, d = 0;
+                for (int r = 0; r < runs; r += 2) {
+                    const int n0 = len[r], n1 = len[r + 1], nn = n0 + n1 < kSortMax ? n0 + n1 : kSortMax;
+                    if (c >= chunks) { // the last pair that starts at or before c (n below: past its end)
+                        pa = base;
+                        na = n0;
+                        nb = n1;
+                        n = nn;
+                        po = out;
+                        d = KO * (c - chunks);
+                    }
+                    base += n0 + n1;
+                    out += nn;
+                    chunks += (nn + KO - 1) / KO;
+                }
+                if (d < n) {
+                    const uint64_t *A = from_ + pa, *B = A + na;
+                    int lo = d > nb ? d - nb : 0, hi = d < na ? d : na;
+                    while (lo < hi) {
+                        const int m = (lo + hi) >> 1;
+                        const bool more = A[m] > B[d - 1 - m];
+                        lo = more ? m + 1 : lo;
+                        hi = more ? hi : m;
+                    }
+                    int i = lo, j = d - lo;
+                    uint64_t x = i < na ? A[i] : 0, y = j < nb ? B[j] : 0;
 #pragma unroll
-            for (int k = 0; k < KPT; ++k) {
-                const int i = k * kSfThreads + int(threadIdx.x);
-                const int r = i / size, at = i % size;
-                if (at < L.len[r]) {
-                    const uint64_t key = from_[i];
-                    const int pos = at + sf_larger(from_ + (r ^ 1) * size, L.len[r ^ 1], key);
-                    if (pos < kSortMax) to[(r >> 1) * 2 * size + pos] = key;
+                    for (int u = 0; u < KO; ++u)
+                        if (d + u < n) {
+                            const bool ta = x > y;
+                            to[po + d + u] = ta ? x : y;
+                            i += ta ? 1 : 0;
+                            j += ta ? 0 : 1;
+                            const uint64_t nx = ta ? (i < na ? A[i] : 0) : (j < nb ? B[j] : 0);
+                            x = ta ? nx : x;
+                            y = ta ? y : nx;
+                        }
+                }
+                if (c0 + kSfThreads >= chunks) { // (uniform)
+                    if (int(threadIdx.x) < runs / 2) {
+                        const int nn = len[2 * threadIdx.x] + len[2 * threadIdx.x + 1];
+                        L.len[cur ^ 1][threadIdx.x] = nn < kSortMax ? nn : kSortMax;
+                    }
+                    total = out;
+                    break;
                 }
             }
             __syncthreads();
-            int n = 0;
-            if (int(threadIdx.x) < runs / 2) n = L.len[2 * threadIdx.x] + L.len[2 * threadIdx.x + 1];
-            __syncthreads();
-            if (int(threadIdx.x) < runs / 2) L.len[threadIdx.x] = n < kSortMax ? n : kSortMax;
-            __syncthreads();
             cur ^= 1;
         }
-        const int64_t ng = L.len[0];
+        const int64_t ng = total;
         if (sf_emit_sorted(L, L.keys[cur], ng, int64_t(nc), S, mx, temperature, top_p, min_p, oi, op, out_n + row))
             return;
         __syncthreads();
