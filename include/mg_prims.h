@@ -216,7 +216,8 @@ int mg_dequant_q8_0(mg_ctx *ctx, const int8_t *qs, const uint16_t *d, void *out,
  * ldo, 0 = q_heads*head_dim). Tile-wise online softmax with bf16
  * probabilities in the p.v product, the reference tier's contract: a
  * numerical envelope, not bits. head_dim 64 or 128; any number of query heads
- * per kv head (groups of more than 8 are served by several work-groups). */
+ * per kv head. Few query tiles over many keys split their keys over the
+ * context's workspace when their partials fit it. */
 int mg_attn_prefill(mg_ctx *ctx, const uint16_t *q, int64_t ldq, const uint16_t *k_cache, const uint16_t *v_cache,
                     int64_t tokens, int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t cache_slots,
                     int64_t pos0, int64_t window, double scaling, float *out, int64_t ldo);
