@@ -365,6 +365,37 @@ def test_sample_rows_split_random(prims, case):
         assert np.abs(probs[r, :n[r]].astype(np.float64) - wp).max() <= 2e-6, (case, r)
 
 
+@pytest.mark.parametrize("rows", (9, 18))
+def test_sample_rows_merge_edges(prims, rows):
+    """runs merged four keys a thread: rows of few candidates and of counts about the
+    chunks, the work-group and the 4096 keys kept, spread over the row or in one slice
+    (the other runs empty)"""
+    import torch
+    rng = np.random.default_rng(80 + rows)
+    V, G = 65536, 16 if rows <= 16 else 8
+    counts = (1, 3, 4, 5, 127, 1025, 4095, 4096, 4097)
+    L = np.full((rows, V), -np.inf, np.float32)
+    one = np.flatnonzero((np.arange(V) // 256) % G == G - 1)
+    for r in range(rows):
+        c = counts[r % 9]
+        at = rng.permutation(one)[:c] if r >= 9 and c <= len(one) else rng.permutation(V)[:c]
+        L[r, at] = rng.standard_normal(c) * 1.5
+    want = O.sample_rows(L, np.argmax(L, axis=1), 0, 1.0, 0.9, 0.0)
+    ids, probs, n = prims.sample_rows(torch.from_numpy(L).cuda(), 0, 1.0, 0.9, 0.0)
+    ids, probs, n = ids.cpu().numpy(), probs.cpu().numpy(), n.cpu().numpy()
+    for r in range(rows):
+        x = np.sort(L[r][np.isfinite(L[r])])[::-1]
+        e32 = np.exp(x - x[0])
+        c32 = np.searchsorted(np.cumsum(e32 / e32.sum()), np.float32(0.9)) + 1
+        c64 = np.searchsorted(np.cumsum(softmax(x.astype(np.float64))), np.float64(np.float32(0.9))) + 1
+        if c32 != c64:
+            continue  # the cut lies within the summation orders' distance
+        wi, wp = want[r]
+        assert n[r] == len(wi), (r, n[r], len(wi))
+        assert np.array_equal(ids[r, :n[r]], wi), r
+        assert np.abs(probs[r, :n[r]].astype(np.float64) - wp).max() <= 2e-6, r
+
+
 @pytest.mark.parametrize("rows,V,sigma", ((2, 201088, 3.0), (17, 201088, 2.5), (3, 16384, 3.0), (5, 16387, 2.5),
                                           (40, 65536, 3.0)))
 def test_sample_rows_uneven_slices(prims, rows, V, sigma):
