@@ -45,42 +45,17 @@
 // reads (0.4), staging (0.25) and the 7 us a work-group starts and ends with.
 #include "mg_device.hpp"
 #include "mg_internal.hpp"
+#include "mg_prefill_plan.hpp"
 
 #include <type_traits>
 
 namespace mg
 {
-    constexpr int kPfKeys = 64;                // keys per step
     constexpr int kPfAhead = 4;                // K fragments read ahead of the products
     constexpr int kPfVAhead = 3;               // V fragments read ahead
 
     // out rows need no more than a float's alignment
     typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-
-    struct PfArgs
-    {
-        int64_t nkv, ldq, ldo, slots, pos0, window;
-        uint32_t npair, hpg, nqt; // T * hpg (row, head) pairs a kv head, heads per kv head, pair tiles
-        uint32_t nfirst;          // shortest tiles that start ahead of the others
-        uint32_t lw;              // log2 of the pairs per tile (work-group)
-        int parts, per;           // key parts per tile, steps per part
-        float scale2;             // |scaling| * log2(e), 2^-126 in place of 0
-        uint32_t qsign;           // 0x80008000 when scaling < 0: q enters with its sign flipped
-    };
-
-    // The keys a pair tile attends: [klo, klo + span], from its first pair's
-    // window start to its last live pair's position
-    struct PfSpan
-    {
-        int64_t klo;
-        int span;
-    };
-    __host__ __device__ inline PfSpan pf_span(int64_t pos0, int64_t window, uint32_t hpg, uint32_t pb0, uint32_t pl)
-    {
-        const int64_t p0 = pos0 + pb0 / hpg;
-        const int64_t klo = window > 0 && p0 - window + 1 > 0 ? p0 - window + 1 : 0;
-        return {klo, int(pos0 + pl / hpg - klo)};
-    }
 
     // W waves of 32 (query row, head) pairs each: pair p of the work-group's kv
     // head is query row p / hpg, head p % hpg, so a wave's columns may mix rows
@@ -478,59 +453,6 @@ namespace mg
         float *dst = out + row * a.ldo + hd * D + d0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) dst[k] = o[k] * inv;
-    }
-
-    // Pairs per tile, parts per tile and steps per part. One 256-pair
-    // work-group a tile leaves CUs idle when the tiles are few: then tiles of
-    // half as many pairs (four waves instead of eight, one a SIMD, a step in
-    // about 0.65 of the time; only in one round, as two of them take longer
-    // than one of 256 pairs) or, behind long contexts (100 tokens of 32 / 2
-    // heads: 26 tiles of 142 steps), the tiles' keys in parts that a second
-    // kernel merges, or both. Priced in 256-pair steps (about 1.8 us): a plan
-    // runs for its longest part times the rounds of work-groups the parts
-    // make; a split adds kMergeSteps for the second launch and the partials'
-    // round trip (D + 2 f32 a pair and part, written and read).
-    inline void pf_plan(PfArgs &a, int cus, int64_t work_bytes, int64_t D)
-    {
-        constexpr double kMergeSteps = 3.0, kBytesPerStep = 8.0e6, kNarrowStep = 0.65;
-        a.parts = 1;
-        a.per = 0;
-        a.nfirst = 0;
-        double best = 0.0;
-        for (uint32_t lw = 8; lw >= 7; --lw) {
-            const uint32_t PW = 1u << lw, nqt = uint32_t((int64_t(a.npair) + PW - 1) >> lw), pl = a.npair - 1;
-            const int64_t tiles = int64_t(nqt) * a.nkv;
-            const double step = lw == 8 ? 1.0 : kNarrowStep;
-            const PfSpan last = pf_span(a.pos0, a.window, a.hpg, (nqt - 1) * PW, pl);
-            const PfSpan first = pf_span(a.pos0, a.window, a.hpg, 0, PW - 1 < pl ? PW - 1 : pl);
-            const int64_t longest = (last.span > first.span ? last.span : first.span) / kPfKeys + 1;
-            const double total = 0.5 * double(tiles) * double((last.span + first.span) / kPfKeys + 2);
-            const double evened = std::ceil(double(tiles) / cus) * total / double(tiles);
-            const double whole = (double(longest) > evened ? double(longest) : evened) * step;
-            if (lw == 8 || (whole < best && tiles <= cus)) {
-                best = whole;
-                a.lw = lw;
-                a.nqt = nqt;
-                a.parts = 1;
-            }
-            if (tiles >= 2 * cus) return; // the tiles fill the chip on their own
-            for (int64_t parts = 2; parts <= 256 && parts <= longest; parts += parts < 16 ? 1 : parts / 8) {
-                const int64_t per = (longest + parts - 1) / parts;
-                const int64_t np = (longest + per - 1) / per;
-                if ((tiles * np << lw) * (D + 2) * int64_t(sizeof(float)) > work_bytes) break;
-                const double some = total / double(per) + 0.5 * double(tiles); // parts holding keys
-                const double live = some < double(tiles * np) ? some : double(tiles * np);
-                const double bytes = 2.0 * live * double(a.npair < PW ? a.npair : PW) * double(D) * 4.0;
-                const double t = double(per) * std::ceil(live / cus) * step + kMergeSteps + bytes / kBytesPerStep;
-                if (t < best && (lw == 8 || live <= cus)) {
-                    best = t;
-                    a.lw = lw;
-                    a.nqt = nqt;
-                    a.parts = int(np);
-                    a.per = int(per);
-                }
-            }
-        }
     }
 
     void launch_attn_prefill(mg_ctx *c, const uint16_t *q, int64_t ldq, const uint16_t *kc, const uint16_t *vc,

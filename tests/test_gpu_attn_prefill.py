@@ -179,3 +179,15 @@ def test_key_split_without_workspace(prims):
     assert float((a - b).abs().max()) <= 2 * TOL
     prefill_case(prims, 20, 40, 8, 128, 3000, 2980, seed=190)
     assert torch.isfinite(a).all()
+
+
+@pytest.mark.parametrize("T,nq,nkv,D,pos0,window", (
+    (57, 32, 2, 128, 986, 1024),
+    (129, 40, 8, 128, 938, 1024),
+    (1606, 1, 1, 128, 0, 542),
+    (130, 8, 1, 64, 950, 1030),
+))
+def test_key_split_window_fills(prims, T, nq, nkv, D, pos0, window):
+    """a window that fills inside the call: the middle tiles attend more keys
+    than the first and the (partial) last one; every row of some heads"""
+    prefill_case(prims, T, nq, nkv, D, pos0 + T, pos0, window=window, seed=200 + T, heads=sorted({0, nq // 2, nq - 1}))
