@@ -20,6 +20,7 @@ namespace mg
     {
         int64_t nkv, ldq, ldo, slots, pos0, window;
         uint32_t npair, hpg, nqt; // T * hpg (row, head) pairs a kv head, heads per kv head, pair tiles
+        uint32_t hw;              // heads of a row's start group (pf_span): hpg's largest divisor <= 8
         uint32_t nfirst;          // shortest tiles that start ahead of the others
         uint32_t lw;              // log2 of the pairs per tile (work-group)
         int parts, per;           // key parts per tile, steps per part
@@ -27,31 +28,39 @@ namespace mg
         uint32_t qsign;           // 0x80008000 when scaling < 0: q enters with its sign flipped
     };
 
-    // The keys a pair tile attends: [klo, klo + span], from its first pair's
-    // window start to its last live pair's position
+    // The keys a pair tile works over: [klo, klo + span], up to its last live
+    // pair's position. With a window klo is the window start of the row that
+    // opens the tile's group of 256 (row, head) pairs, `hw` heads a row: a row's
+    // 64-key steps, and with them its weights' reference (k_attn_prefill), then
+    // lie the same whatever tile width and key parts a call takes. (16 or 24 rows
+    // ahead of the tile for 16 heads a row, 26 for 5 and 128 for one where tiles
+    // are narrow: no step more of 17 at a 1024-key window, two for one head a row.)
     struct PfSpan
     {
         int64_t klo;
         int span;
     };
-    MG_PP PfSpan pf_span(int64_t pos0, int64_t window, uint32_t hpg, uint32_t pb0, uint32_t pl)
+    MG_PP PfSpan pf_span(int64_t pos0, int64_t window, uint32_t hpg, uint32_t hw, uint32_t pb0, uint32_t pl)
     {
-        const int64_t p0 = pos0 + pb0 / hpg;
+        const uint32_t row = pb0 / hpg, at = row * hw + (pb0 - row * hpg) % hw;
+        const int64_t p0 = pos0 + (at & ~255u) / hw;
         const int64_t klo = window > 0 && p0 - window + 1 > 0 ? p0 - window + 1 : 0;
         return {klo, int(pos0 + pl / hpg - klo)};
     }
 
     // The most any tile of PW pairs reaches past its first key (a bound on
-    // pf_span's span). Without a window that is the last position. With one, a
-    // tile's rows past its first add to the window's keys: PW pairs from any
-    // pair of a row on lie in at most (PW + hpg - 2) / hpg rows past the first.
-    // (The end tiles alone do not give it: the first may start before the window
-    // fills, the last may hold few rows.)
-    inline int64_t pf_longest(int64_t pos0, int64_t window, uint32_t hpg, uint32_t npair, uint32_t PW)
+    // pf_span's span). Without a window that is the last position. With one, the
+    // tile's rows add to the window's keys: its own PW pairs, from any pair of a
+    // row on, lie in at most (PW + hpg - 2) / hpg rows past its first, and its
+    // group opens less than 256 / hw rows ahead of that. (The end tiles alone do
+    // not give it: the first may start before the window fills, the last may hold
+    // few rows.)
+    inline int64_t pf_longest(int64_t pos0, int64_t window, uint32_t hpg, uint32_t hw, uint32_t npair, uint32_t PW)
     {
         const int64_t T = int64_t(npair) / hpg, last = pos0 + T - 1;
         if (window <= 0 || window > last) return last;
-        const int64_t rows = (int64_t(PW) + hpg - 2) / hpg;
+        const int64_t ahead = PW == 256 && hw == hpg ? 0 : (254 + int64_t(hw)) / hw; // such tiles are the groups
+        const int64_t rows = (int64_t(PW) + hpg - 2) / hpg + ahead;
         const int64_t most = window - 1 + (rows < T - 1 ? rows : T - 1);
         return most < last ? most : last;
     }
@@ -72,14 +81,16 @@ namespace mg
         a.parts = 1;
         a.per = 0;
         a.nfirst = 0;
+        a.hw = a.hpg;
+        while (a.hw > 8 || a.hpg % a.hw != 0) --a.hw;
         double best = 0.0;
         for (uint32_t lw = 8; lw >= 7; --lw) {
             const uint32_t PW = 1u << lw, nqt = uint32_t((int64_t(a.npair) + PW - 1) >> lw), pl = a.npair - 1;
             const int64_t tiles = int64_t(nqt) * a.nkv;
             const double step = lw == 8 ? 1.0 : kNarrowStep;
-            const PfSpan last = pf_span(a.pos0, a.window, a.hpg, (nqt - 1) * PW, pl);
-            const PfSpan first = pf_span(a.pos0, a.window, a.hpg, 0, PW - 1 < pl ? PW - 1 : pl);
-            const int64_t longest = pf_longest(a.pos0, a.window, a.hpg, a.npair, PW) / kPfKeys + 1;
+            const PfSpan last = pf_span(a.pos0, a.window, a.hpg, a.hw, (nqt - 1) * PW, pl);
+            const PfSpan first = pf_span(a.pos0, a.window, a.hpg, a.hw, 0, PW - 1 < pl ? PW - 1 : pl);
+            const int64_t longest = pf_longest(a.pos0, a.window, a.hpg, a.hw, a.npair, PW) / kPfKeys + 1;
             const double total = 0.5 * double(tiles) * double((last.span + first.span) / kPfKeys + 2);
             const double evened = std::ceil(double(tiles) / cus) * total / double(tiles);
             const double whole = (double(longest) > evened ? double(longest) : evened) * step;

@@ -16,10 +16,13 @@ static bool bad_plan(const mg::PfArgs &a, int64_t work, int64_t D)
     const uint32_t PW = 1u << a.lw;
     if (int64_t(a.nqt) * PW < a.npair || int64_t(a.nqt - 1) * PW >= a.npair) return true;
     if (a.parts > 1 && (int64_t(a.nqt) * a.nkv * a.parts << a.lw) * (D + 2) * 4 > work) return true;
-    const int64_t longest = mg::pf_longest(a.pos0, a.window, a.hpg, a.npair, PW);
+    const int64_t longest = mg::pf_longest(a.pos0, a.window, a.hpg, a.hw, a.npair, PW);
     for (uint32_t qt = 0; qt < a.nqt; ++qt) {
         const uint32_t pb0 = qt << a.lw, pl = (pb0 + PW < a.npair ? pb0 + PW : a.npair) - 1;
-        const mg::PfSpan s = mg::pf_span(a.pos0, a.window, a.hpg, pb0, pl);
+        const mg::PfSpan s = mg::pf_span(a.pos0, a.window, a.hpg, a.hw, pb0, pl);
+        // rows of other tiles' windows may open the keys, but none the call does not attend
+        const int64_t lo0 = a.window > 0 && a.pos0 - a.window + 1 > 0 ? a.pos0 - a.window + 1 : 0;
+        if (s.klo < lo0 || (a.window > 0 && s.klo > a.pos0 + pb0 / a.hpg - a.window + 1 && s.klo > 0)) return true;
         if (s.span < 0 || s.span > longest) return true;
         if (a.parts > 1 && s.span / mg::kPfKeys >= int64_t(a.parts) * a.per) return true;
     }

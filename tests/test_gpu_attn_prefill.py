@@ -191,3 +191,31 @@ def test_key_split_window_fills(prims, T, nq, nkv, D, pos0, window):
     """a window that fills inside the call: the middle tiles attend more keys
     than the first and the (partial) last one; every row of some heads"""
     prefill_case(prims, T, nq, nkv, D, pos0 + T, pos0, window=window, seed=200 + T, heads=sorted({0, nq // 2, nq - 1}))
+
+
+@pytest.mark.parametrize("T,nq,nkv,D,pos0,window", (
+    (100, 32, 2, 128, 9000, 0),
+    (64, 8, 8, 64, 3000, 0),
+    (129, 40, 8, 128, 938, 1024),
+    (57, 32, 2, 128, 986, 1024),    # tiles of 16 or 8 rows in groups of 32
+    (300, 2, 2, 128, 5000, 2000),   # 256 rows a tile: rows whose keys start four steps in
+))
+def test_key_split_rounds_the_same_weights(prims, T, nq, nkv, D, pos0, window):
+    """Split or not, a pair's weights start from one reference, so bf16 rounds the
+    same numbers and a row's output does not depend on how its call is cut: only
+    f32 sums differ, a chain of some 600 additions of 2^-25 rms each (1.5e-6 by a
+    random walk, gated at 2e-5). Weights rounded against another reference are 2e-3
+    apart. (No reference moves here: scores of std 1 stay within 8 of the first
+    step's maximum.)"""
+    import mgprims
+    import torch
+    small = mgprims.Prims(0, workspace_bytes=4096)
+    q = to_dev(O.normal(210, (T, nq, D), 0.0, 1.0, BF16), BF16)
+    k = to_dev(O.normal(211, (pos0 + T, nkv, D), 0.0, 1.0, BF16), BF16)
+    v = to_dev(O.normal(212, (pos0 + T, nkv, D), 0.0, 1.0, BF16), BF16)
+    a = small.attn_prefill(q, k, v, pos0, 1.0 / math.sqrt(D), window)
+    b = prims.attn_prefill(q, k, v, pos0, 1.0 / math.sqrt(D), window)
+    again = prims.attn_prefill(q, k, v, pos0, 1.0 / math.sqrt(D), window)
+    small.close()
+    assert torch.equal(b, again)
+    assert float((a - b).norm() / a.norm()) < 2e-5
