@@ -337,11 +337,10 @@ namespace mg
         }
     }
 
-    // the wave's share of a loaded row: scores (capped, masked) to 2^(s c2 - mc),
-    // mc = the wave's maximum times c2 (rounded); returns the maximum (-inf: no
-    // key with a weight) and the wave's sum
+    // the wave's share of a loaded row as scores (capped, masked keys of partly
+    // visible chunks -inf); returns their maximum (-inf: none, or NaN scores only)
     template <int CH, int WPR, bool CAP>
-    MG_DEV float fast_exp(const SmArgs &a, float c2, int lane, int w, FastRow<CH> &r, float &sum, double *tab)
+    MG_DEV float fast_scores(const SmArgs &a, int lane, int w, FastRow<CH> &r, double *tab)
     {
         [[maybe_unused]] CapTab ct{tab, false};
         const int lo = int(r.lo64), hi = int(r.hi64);
@@ -368,23 +367,28 @@ namespace mg
 #pragma unroll
             for (int e = 0; e < 8; ++e) m = __builtin_fmaxf(m, r.v[c][e]);
         }
-        m = dpp_max(m);
-        sum = 0.0f;
-        if (m != kNegInf) {
-            const float mc = m * c2;
+        return dpp_max(m);
+    }
+
+    // those scores to 2^(s c2 - mc); returns the wave's sum. mc = the maximum
+    // times c2, rounded, and 0 where the maximum is -inf: -inf scores then weigh
+    // 0 and a NaN one, which no maximum shows, still reaches the sum
+    template <int CH, int WPR>
+    MG_DEV float fast_exp(float c2, float mc, int w, FastRow<CH> &r)
+    {
+        const int lo = int(r.lo64), hi = int(r.hi64);
+        float sum = 0.0f;
 #pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                const int cb = (c * WPR + w) * 512;
-                if (cb > hi || cb + 511 < lo) continue;
+        for (int c = 0; c < CH; ++c) {
+            const int cb = (c * WPR + w) * 512;
+            if (cb > hi || cb + 511 < lo) continue;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    r.v[c][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(r.v[c][e], c2, -mc)); // masked: exp2(-inf) = 0
-                    sum += r.v[c][e];
-                }
+            for (int e = 0; e < 8; ++e) {
+                r.v[c][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(r.v[c][e], c2, -mc));
+                sum += r.v[c][e];
             }
         }
-        sum = dpp_sum_f32(sum);
-        return m;
+        return dpp_sum_f32(sum);
     }
 
     // the wave's share of the row times `f` to storage; chunks without a visible
@@ -436,8 +440,8 @@ namespace mg
         fast_load<CH, 1>(a, x, row, lane, 0, r);
         if (!r.live) return;
         __shared__ double tab[CAP ? 128 : 1];
-        float sum;
-        const float m = fast_exp<CH, 1, CAP>(a, c2, lane, 0, r, sum, tab);
+        const float m = fast_scores<CH, 1, CAP>(a, lane, 0, r, tab);
+        const float sum = fast_exp<CH, 1>(c2, m == kNegInf ? 0.0f : m * c2, 0, r);
         // a row with non-finite sums is redone on the accurate path
         if (m != kNegInf && !(sum < __builtin_huge_valf())) {
             softmax_row_accurate<SF32, SO, CH, CAP>(a, x + row * a.ldx, y + row * a.ldy, r.lo64, r.hi64, VEC, lane);
@@ -450,12 +454,10 @@ namespace mg
     // their registers: one read and one write of HBM, where the split passes
     // below read the scores twice (40 heads of 1000 queries over 4000 keys: 254 ->
     // 143 us, 6.2 TB/s of the visible scores and the probabilities; 40 decode rows
-    // of 16384: 11.3 -> 7.4, a launch less). Bound by HBM. Each wave takes its own maximum and sum;
-    // the waves meet once, in LDS, and the move to the row's maximum goes into
-    // each wave's factor: 2^(mc_w - mc) / L, from the rounded maxima mc the
-    // exponents used, so their roundings cancel as within one wave.
+    // of 16384: 11.3 -> 7.4, a launch less). Bound by HBM. The waves meet in LDS
+    // twice, for the row's maximum and for its sum.
     // A row with NaN or infinite scores gets NaN at every visible key (its sum
-    // is NaN) and zeros at the masked ones, as in the split passes.
+    // is NaN, whichever wave holds them) and zeros at the masked ones.
     template <class SO, int WPR, bool CAP, bool VEC>
     __global__ __launch_bounds__(64 * WPR) void k_softmax_group(const float *__restrict__ x,
                                                                 typename SO::raw *__restrict__ y, SmArgs a, float c2)
@@ -468,29 +470,25 @@ namespace mg
         FastRow<CH> r;
         fast_load<CH, WPR>(a, x, row, lane, w, r);
         __shared__ double tab[CAP ? 128 * WPR : 1];
-        float sum;
-        const float m = fast_exp<CH, WPR, CAP>(a, c2, lane, w, r, sum, tab + (CAP ? 128 * w : 0));
-        if (lane == 0) {
-            red[w] = m;
-            red[WPR + w] = sum;
-        }
+        const float m = fast_scores<CH, WPR, CAP>(a, lane, w, r, tab + (CAP ? 128 * w : 0));
+        if (lane == 0) red[w] = m;
         __syncthreads();
         float M = red[0];
 #pragma unroll
         for (int i = 1; i < WPR; ++i) M = __builtin_fmaxf(M, red[i]);
-        const float Mc = M * c2;
+        const float sum = fast_exp<CH, WPR>(c2, M == kNegInf ? 0.0f : M * c2, w, r);
+        if (lane == 0) red[WPR + w] = sum;
+        __syncthreads();
         float L = 0.0f;
 #pragma unroll
-        for (int i = 0; i < WPR; ++i)
-            if (red[i] != kNegInf) L += red[WPR + i] * __builtin_amdgcn_exp2f(red[i] * c2 - Mc);
-        if (M != kNegInf && !(L < __builtin_huge_valf())) {
+        for (int i = 0; i < WPR; ++i) L += red[WPR + i];
+        if (!(L < __builtin_huge_valf())) {
             ro *yr = y + row * a.ldy;
             for (int j = int(threadIdx.x); j < int(a.kc); j += 64 * WPR)
                 yr[j] = j >= int(r.lo64) && j <= int(r.hi64) ? SO::enc32(__builtin_nanf("")) : ro(0);
             return;
         }
-        const float f = m == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(m * c2 - Mc) * __builtin_amdgcn_rcpf(L);
-        fast_store<SO, CH, WPR, VEC>(a, y, row, f, m == kNegInf, lane, w, r);
+        fast_store<SO, CH, WPR, VEC>(a, y, row, __builtin_amdgcn_rcpf(L), M == kNegInf, lane, w, r);
     }
 
     // ------------------------------------------------------------- split rows

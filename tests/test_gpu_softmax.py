@@ -318,3 +318,41 @@ def test_group_rows_nonfinite(prims, kc):
         e = np.where(vis[0, r], np.exp(xr - xr[vis[0, r]].max()), 0.0)
         d = ulp_diff16(O.from_f64(y[0, r].astype(np.float64), BF16), O.from_f64(e / e.sum(), BF16))
         assert d.max() <= 1, r
+
+
+def scores_case(prims, x, q_pos0, softcap=0.0, dt_out=BF16, mask=O.MASK_CAUSAL, window=0):
+    """f32 scores x [1, q, kc] through softmax_rows, and the oracle's result: as
+    16-bit patterns (NaN canonical in both)"""
+    import torch
+    dy = torch.full(x.shape, 7.0, dtype=torch.bfloat16 if dt_out == BF16 else torch.float16, device="cuda:0")
+    prims.softmax_rows(torch.from_numpy(x).cuda(), dy, SCALE, mask, window, q_pos0, softcap)
+    ref = O.softmax_rows(x.astype(np.float64), SCALE, mask, window, q_pos0, softcap, F32, O.F64)
+    return from_dev(dy, dt_out), O.from_f64(ref, dt_out)
+
+
+def check_nan_rows(y, ref, dt_out=BF16):
+    """NaN exactly where the oracle has it, the rest within an ulp"""
+    from util import is_nan16
+    nan = is_nan16(ref, dt_out)
+    assert nan.any()
+    assert np.array_equal(is_nan16(y, dt_out), nan)
+    assert ulp_diff16(y[~nan], ref[~nan]).max() <= 1
+
+
+@pytest.mark.parametrize("softcap", (0.0, 30.0))
+@pytest.mark.parametrize("kc", (2049, 4096, 4097, 8192, 10001, 16384))
+def test_group_rows_nan_alone_in_its_wave(prims, kc, softcap):
+    """NaN scores that no wave's maximum shows: a row of NaN only, a row whose
+    last wave with a visible key has that one key, NaN (waves take 512-key chunks
+    in turn, two, four or eight a row), and a wave of NaN and -inf"""
+    q = 4
+    x = O.to_f64(O.normal(15, (1, q, kc), 0.0, 3.0, F32), F32).astype(np.float32)
+    x[0, 0, :] = np.nan                      # sees keys 0..512
+    x[0, 1, 513] = np.nan                    # its last key, beside key 512 of the same wave
+    x[0, 1, 512] = -np.inf if softcap == 0.0 else np.nan
+    x[0, 2, 600:] = np.nan                   # past its keys: untouched
+    check_nan_rows(*scores_case(prims, x, 512, softcap))
+    x = O.to_f64(O.normal(16, (1, q, kc), 0.0, 3.0, F32), F32).astype(np.float32)
+    x[0, 0, 1024] = np.nan                   # its only key in the third chunk
+    x[0, 3, :] = np.nan
+    check_nan_rows(*scores_case(prims, x, 1024, softcap))
