@@ -248,12 +248,15 @@ namespace mg
                 sum += double(s[c][e]);
             }
         sum = wave_sum(sum);
+        const bool nan = sum != sum; // NaN or +inf scores: NaN at the visible keys, 0 at the others
         const float inv = m == kNegInf ? 0.0f : float(1.0 / sum);
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
+            const int64_t j0 = int64_t(lane + 64 * c) * 8;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) s[c][e] *= inv;
-            store_probs<SO>(a, yr, int64_t(lane + 64 * c) * 8, vec, s[c]);
+            for (int e = 0; e < 8; ++e)
+                s[c][e] = !nan ? s[c][e] * inv : j0 + e >= lo && j0 + e <= hi ? __builtin_nanf("") : 0.0f;
+            store_probs<SO>(a, yr, j0, vec, s[c]);
         }
     }
 
@@ -442,8 +445,9 @@ namespace mg
         __shared__ double tab[CAP ? 128 : 1];
         const float m = fast_scores<CH, 1, CAP>(a, lane, 0, r, tab);
         const float sum = fast_exp<CH, 1>(c2, m == kNegInf ? 0.0f : m * c2, 0, r);
-        // a row with non-finite sums is redone on the accurate path
-        if (m != kNegInf && !(sum < __builtin_huge_valf())) {
+        // a row with non-finite sums is redone on the accurate path (NaN scores only:
+        // the maximum is -inf, the sum NaN)
+        if (!(sum < __builtin_huge_valf())) {
             softmax_row_accurate<SF32, SO, CH, CAP>(a, x + row * a.ldx, y + row * a.ldy, r.lo64, r.hi64, VEC, lane);
             return;
         }

@@ -336,7 +336,7 @@ def check_nan_rows(y, ref, dt_out=BF16):
     nan = is_nan16(ref, dt_out)
     assert nan.any()
     assert np.array_equal(is_nan16(y, dt_out), nan)
-    assert ulp_diff16(y[~nan], ref[~nan]).max() <= 1
+    assert np.all(ulp_diff16(y[~nan], ref[~nan]) <= 1)
 
 
 @pytest.mark.parametrize("softcap", (0.0, 30.0))
@@ -356,3 +356,34 @@ def test_group_rows_nan_alone_in_its_wave(prims, kc, softcap):
     x[0, 0, 1024] = np.nan                   # its only key in the third chunk
     x[0, 3, :] = np.nan
     check_nan_rows(*scores_case(prims, x, 1024, softcap))
+
+
+@pytest.mark.parametrize("softcap", (0.0, 30.0))
+@pytest.mark.parametrize("kc", (1, 64, 500, 512, 1000, 2047, 2048))
+def test_short_rows_of_nan(prims, kc, softcap):
+    """rows of up to 2048 keys whose visible scores are all NaN, or NaN and -inf:
+    NaN at the visible keys, 0 at the masked ones; beside them a row with one NaN"""
+    q = min(4, kc)
+    x = O.to_f64(O.normal(17, (1, q, kc), 0.0, 3.0, F32), F32).astype(np.float32)
+    x[0, 0, :] = np.nan
+    if q == 4:
+        x[0, 1, ::2] = np.nan
+        x[0, 1, 1::2] = -np.inf if softcap == 0.0 else np.nan
+        x[0, 2, 7] = np.nan
+    check_nan_rows(*scores_case(prims, x, kc // 2, softcap))
+
+
+@pytest.mark.parametrize("dt_in,dt_out", ((BF16, BF16), (F32, F32)))
+def test_accurate_rows_of_nan(prims, dt_in, dt_out):
+    """the same through the accurate one-wave kernel (16-bit scores, f32 probabilities)"""
+    x = O.to_f64(O.normal(18, (1, 4, 700), 0.0, 3.0, dt_in), dt_in)
+    x[0, 0, :] = np.nan
+    x[0, 1, ::2] = np.nan
+    x[0, 1, 1::2] = -np.inf
+    x[0, 2, 7] = np.nan
+    dy = to_dev(np.zeros((1, 4, 700), np.float32 if dt_out == F32 else np.uint16), dt_out)
+    prims.softmax_rows(to_dev(O.from_f64(x, dt_in), dt_in), dy, SCALE, O.MASK_CAUSAL, 0, 300)
+    y = O.to_f64(from_dev(dy, dt_out), dt_out)
+    ref = O.softmax_rows(x, SCALE, O.MASK_CAUSAL, 0, 300, 0.0, dt_in, O.F64)
+    assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.isnan(ref[0, :3]).any(-1).all()
+    assert np.all(y[0, :, 304:] == 0.0)
