@@ -223,6 +223,13 @@ namespace mg
         }
     }
 
+    // 8 keys of a row with NaN or +inf scores: NaN where visible, 0 where masked
+    MG_DEV void nan_row8(float *p, int64_t j0, int64_t lo, int64_t hi)
+    {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[e] = j0 + e >= lo && j0 + e <= hi ? __builtin_nanf("") : 0.0f;
+    }
+
     // --------------------------------------------------------- one wave per row
     // Accurate row: transformed scores, exp of the exactly formed s - max, f64
     // sum, one rounding at the output. Lane `lane` owns keys 8*(lane + 64c) + e.
@@ -248,14 +255,14 @@ namespace mg
                 sum += double(s[c][e]);
             }
         sum = wave_sum(sum);
-        const bool nan = sum != sum; // NaN or +inf scores: NaN at the visible keys, 0 at the others
+        const bool nan = sum != sum; // NaN or +inf scores
         const float inv = m == kNegInf ? 0.0f : float(1.0 / sum);
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
             const int64_t j0 = int64_t(lane + 64 * c) * 8;
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                s[c][e] = !nan ? s[c][e] * inv : j0 + e >= lo && j0 + e <= hi ? __builtin_nanf("") : 0.0f;
+            for (int e = 0; e < 8; ++e) s[c][e] *= inv;
+            if (nan) nan_row8(s[c], j0, lo, hi);
             store_probs<SO>(a, yr, j0, vec, s[c]);
         }
     }
@@ -538,12 +545,12 @@ namespace mg
             for (int e = 0; e < 8; ++e) m = s[c][e] > m ? s[c][e] : m;
         }
         m = block_max_f32(m, red);
+        // (a chunk of NaN scores alone keeps m = -inf and sums to NaN)
         double sum = 0.0;
-        if (m != kNegInf)
 #pragma unroll
-            for (int c = 0; c < 2; ++c)
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) sum += s[c][e] == kNegInf ? 0.0 : double(exp_diff(s[c][e], m));
+            for (int e = 0; e < 8; ++e) sum += s[c][e] == kNegInf ? 0.0 : double(exp_diff(s[c][e], m));
         sum = block_sum_f64(sum, redd);
         if (threadIdx.x == 0) part[row * gridDim.x + blockIdx.x] = make_float2(m, float(sum));
     }
@@ -576,9 +583,8 @@ namespace mg
         for (int i = threadIdx.x; i < nch; i += blockDim.x) M = pr[i].x > M ? pr[i].x : M;
         M = block_max_f32(M, red);
         double L = 0.0;
-        if (M != kNegInf)
-            for (int i = threadIdx.x; i < nch; i += blockDim.x)
-                if (pr[i].x != kNegInf) L += double(pr[i].y) * mgm::exp(double(pr[i].x) - double(M));
+        for (int i = threadIdx.x; i < nch; i += blockDim.x) // a maximum of -inf: a sum of 0 or NaN
+            L += pr[i].x == kNegInf ? double(pr[i].y) : double(pr[i].y) * mgm::exp(double(pr[i].x) - double(M));
         L = block_sum_f64(L, redd);
         const float inv = M == kNegInf ? 0.0f : float(1.0 / L);
 #pragma unroll
@@ -586,6 +592,7 @@ namespace mg
             const int64_t j0 = base + int64_t(threadIdx.x + 256 * c) * 8;
 #pragma unroll
             for (int e = 0; e < 8; ++e) s[c][e] = s[c][e] == kNegInf ? 0.0f : exp_diff(s[c][e], M) * inv;
+            if (L != L) nan_row8(s[c], j0, lo, hi);
             store_probs<SO>(a, yr, j0, vec, s[c]);
         }
     }
@@ -661,12 +668,12 @@ namespace mg
             for (int e = 0; e < 8; ++e) m = t[c][e] > m ? t[c][e] : m;
         }
         m = block_max_dpp(m, red);
+        const float ref = m == kNegInf ? 0.0f : m; // NaN scores alone: the sum is NaN
         float sum = 0.0f;
-        if (m != kNegInf)
 #pragma unroll
-            for (int c = 0; c < 2; ++c)
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) sum += __builtin_amdgcn_exp2f(t[c][e] - m); // exp2(-inf) = 0
+            for (int e = 0; e < 8; ++e) sum += __builtin_amdgcn_exp2f(t[c][e] - ref); // exp2(-inf) = 0
         sum = block_sum_dpp(sum, red);
         if (threadIdx.x == 0) part[row * gridDim.x + blockIdx.x] = make_float2(m, sum);
     }
@@ -694,16 +701,17 @@ namespace mg
         for (int i = threadIdx.x; i < nch; i += blockDim.x) M = pr[i].x > M ? pr[i].x : M;
         M = block_max_dpp(M, red);
         float L = 0.0f;
-        if (M != kNegInf)
-            for (int i = threadIdx.x; i < nch; i += blockDim.x)
-                if (pr[i].x != kNegInf) L += pr[i].y * __builtin_amdgcn_exp2f(pr[i].x - M);
+        for (int i = threadIdx.x; i < nch; i += blockDim.x) // a maximum of -inf: a sum of 0 or NaN
+            L += pr[i].x == kNegInf ? pr[i].y : pr[i].y * __builtin_amdgcn_exp2f(pr[i].x - M);
         L = block_sum_dpp(L, red);
         const float inv = M == kNegInf ? 0.0f : 1.0f / L;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
+            const int64_t j0 = base + int64_t(threadIdx.x + 256 * c) * 8;
 #pragma unroll
             for (int e = 0; e < 8; ++e) t[c][e] = t[c][e] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(t[c][e] - M) * inv;
-            store_probs<SO>(a, yr, base + int64_t(threadIdx.x + 256 * c) * 8, vec, t[c]);
+            if (L != L) nan_row8(t[c], j0, lo, hi);
+            store_probs<SO>(a, yr, j0, vec, t[c]);
         }
     }
 
@@ -738,12 +746,12 @@ namespace mg
                 m = __builtin_fmaxf(m, t[c][e]);
             }
         m = block_max_dpp(m, red);
+        const float ref = m == kNegInf ? 0.0f : m; // NaN scores alone: the sum is NaN
         float sum = 0.0f;
-        if (m != kNegInf)
 #pragma unroll
-            for (int c = 0; c < 4; ++c)
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) sum += __builtin_amdgcn_exp2f(t[c][e] - m); // exp2(-inf) = 0
+            for (int e = 0; e < 4; ++e) sum += __builtin_amdgcn_exp2f(t[c][e] - ref); // exp2(-inf) = 0
         sum = block_sum_dpp(sum, red);
         if (threadIdx.x == 0) part[row * gridDim.x + blockIdx.x] = make_float2(m, sum);
     }
@@ -780,21 +788,20 @@ namespace mg
         float M = pm;
         for (int i = threadIdx.x + blockDim.x; i < nch; i += blockDim.x) M = pr[i].x > M ? pr[i].x : M;
         M = block_max_dpp(M, red);
-        float L = 0.0f;
-        if (M != kNegInf) {
-            if (pm != kNegInf) L = pl * __builtin_amdgcn_exp2f(pm - M);
-            for (int i = threadIdx.x + blockDim.x; i < nch; i += blockDim.x)
-                if (pr[i].x != kNegInf) L += pr[i].y * __builtin_amdgcn_exp2f(pr[i].x - M);
-        }
+        // a maximum of -inf: a sum of 0 or NaN
+        float L = !own ? 0.0f : pm == kNegInf ? pl : pl * __builtin_amdgcn_exp2f(pm - M);
+        for (int i = threadIdx.x + blockDim.x; i < nch; i += blockDim.x)
+            L += pr[i].x == kNegInf ? pr[i].y : pr[i].y * __builtin_amdgcn_exp2f(pr[i].x - M);
         L = block_sum_dpp(L, red);
-        const float inv = M == kNegInf ? 0.0f : 1.0f / L;
+        const float inv = L != L ? L : M == kNegInf ? 0.0f : 1.0f / L;
+        const float ref = M == kNegInf ? 0.0f : M;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             Vec<ro, 8> o; // elements 0..3 stored (8 bytes), 4..7 unused
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int j = base + 1024 * c + e;
-                const float p = (j >= lo && j <= hi) ? __builtin_amdgcn_exp2f(u[c].v[e] * c2 - M) * inv : 0.0f;
+                const float p = (j >= lo && j <= hi) ? __builtin_amdgcn_exp2f(u[c].v[e] * c2 - ref) * inv : 0.0f;
                 o.v[e] = SO::enc32(p);
             }
             const Vec<uint32_t, 4> w = __builtin_bit_cast(Vec<uint32_t, 4>, o);

@@ -387,3 +387,26 @@ def test_accurate_rows_of_nan(prims, dt_in, dt_out):
     ref = O.softmax_rows(x, SCALE, O.MASK_CAUSAL, 0, 300, 0.0, dt_in, O.F64)
     assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.isnan(ref[0, :3]).any(-1).all()
     assert np.all(y[0, :, 304:] == 0.0)
+
+
+@pytest.mark.parametrize("dt_in,dt_out,kc,softcap", (
+    (F32, BF16, 20000, 0.0), (F32, BF16, 20001, 0.0), (F32, F32, 5000, 0.0), (F32, BF16, 20000, 30.0)))
+def test_split_rows_of_nan(prims, dt_in, dt_out, kc, softcap):
+    """rows split over work-groups of 4096 keys: NaN scores only, a chunk whose one
+    visible key is NaN, a chunk of NaN and -inf beside finite ones, and a row of
+    -inf only (zeros: no key has weight)"""
+    x = O.to_f64(O.normal(19, (1, 5, kc), 0.0, 3.0, dt_in), dt_in)
+    x[0, 0, :] = np.nan                                      # sees keys 0..4096
+    x[0, 1, 4096:] = np.nan                                  # sees two keys of the second chunk
+    x[0, 2, 4096] = np.nan
+    x[0, 2, 4097:] = -np.inf if softcap == 0.0 else np.nan
+    x[0, 3, :] = -np.inf
+    dy = to_dev(np.zeros((1, 5, kc), np.float32 if dt_out == F32 else np.uint16), dt_out)
+    prims.softmax_rows(to_dev(O.from_f64(x, dt_in), dt_in), dy, SCALE, O.MASK_CAUSAL, 0, 4096, softcap)
+    y = O.to_f64(from_dev(dy, dt_out), dt_out)
+    ref = O.softmax_rows(x, SCALE, O.MASK_CAUSAL, 0, 4096, softcap, dt_in, O.F64)
+    if softcap == 0.0:
+        ref[0, 3] = 0.0
+    assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.isnan(ref[0, :3]).any(-1).all()
+    ok = ~np.isnan(ref) & (ref > 1e-30)
+    assert np.abs(y[ok] / ref[ok] - 1.0).max() < 2.0 ** -7
