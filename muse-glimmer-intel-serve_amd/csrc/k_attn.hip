@@ -166,6 +166,9 @@ namespace mg
             }
             mx = rows4_max(mx);
             const float mn = __builtin_fmaxf(m, mx);
+            // no score above -inf yet: a zero reference, so that -inf scores weigh 0
+            // and only NaN ones reach the sum
+            const float mref = mn == -__builtin_huge_valf() ? 0.0f : mn;
             // P as A of the P V product: element 4t + r of lane (head n, c) is key 16 t + 4c + r
             bf16x8 phi, plo;
             float ps = 0.0f;
@@ -173,7 +176,7 @@ namespace mg
             for (int t = 0; t < 2; ++t)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float p = __builtin_amdgcn_exp2f(sc[t][r] - mn);
+                    const float p = __builtin_amdgcn_exp2f(sc[t][r] - mref);
                     ps += p;
                     const __bf16 hi = __bf16(p);
                     phi[4 * t + r] = hi;
@@ -182,7 +185,7 @@ namespace mg
             if (__builtin_amdgcn_ballot_w64(mn != m) != 0) {
                 // some head's running max moved: rescale its sum and its O row
                 // (rows are heads 4c + r; their factors come from lanes 4c + r)
-                const float corr = __builtin_amdgcn_exp2f(m - mn); // first step: 2^-inf = 0
+                const float corr = __builtin_amdgcn_exp2f(m - mref); // first step: 2^-inf = 0
                 l *= corr;
                 float cr[4];
 #pragma unroll
@@ -229,7 +232,8 @@ namespace mg
 
     // merge the splits of one query head for 16 of its dims (one work-group
     // per (head, 16 dims)): M = max m_s, weights 2^(m_s - M),
-    // out = sum_s w_s acc_s / sum_s w_s l_s. Thread 16 sg + d takes dim d of
+    // out = sum_s w_s acc_s / sum_s w_s l_s. A split whose maximum is -inf holds
+    // nothing (sum 0) or NaN scores only, and its NaN enters. Thread 16 sg + d takes dim d of
     // splits sg, sg + 16, ...; the 16 partial sums are added in LDS.
     __global__ __launch_bounds__(256) void k_attn_combine(const float *__restrict__ pm, const float *__restrict__ pl,
                                                           const float *__restrict__ pa, float *__restrict__ out,
@@ -250,7 +254,7 @@ namespace mg
         M = __builtin_fmaxf(__builtin_fmaxf(redm[0], redm[1]), __builtin_fmaxf(redm[2], redm[3]));
         double L = 0.0;
         for (int s = tid; s < nsplit; s += 256)
-            if (mh[s] != -__builtin_huge_valf()) L += double(__builtin_amdgcn_exp2f(mh[s] - M)) * double(lh[s]);
+            if (mh[s] != -__builtin_huge_valf() || lh[s] != lh[s]) L += double(__builtin_amdgcn_exp2f(mh[s] - M)) * double(lh[s]);
         L = dpp_sum(L);
         if (lane == 0) redl[wv] = L;
         // the 16 output dims: each thread takes whole splits (64 contiguous
@@ -261,7 +265,7 @@ namespace mg
         for (int e = 0; e < 16; ++e) o[e] = 0.0f;
         for (int s = tid; s < nsplit; s += 256) {
             const float ms = mh[s];
-            if (ms != -__builtin_huge_valf()) {
+            if (ms != -__builtin_huge_valf() || lh[s] != lh[s]) {
                 const float wgt = __builtin_amdgcn_exp2f(ms - M);
                 const Vec<float, 4> *src = reinterpret_cast<const Vec<float, 4> *>(pa + (h * nsplit + s) * D + d0);
 #pragma unroll

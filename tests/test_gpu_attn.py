@@ -123,3 +123,41 @@ def test_small_workspace_takes_the_longer_splits(prims):
     small = mgprims.Prims(0, workspace_bytes=8 * 8 * (2 + 128) * 4)
     attn_case(small, 8, 2, 128, 2048, 2047, seed=98)
     small.close()
+
+
+@pytest.mark.parametrize("keys", (1, 20, 65, 1025, 20001))
+def test_nan_key_alone_in_its_split(prims, keys):
+    """The newest key of one kv head is NaN and alone in the last split (64-key
+    splits, 256-key ones past 256 of them, a single split): the head group's outputs are NaN, the
+    others as ever; and a key of score -inf there weighs nothing, also where the
+    whole first step has only such scores"""
+    nq, nkv, D = 40, 8, 128
+    q = np.abs(O.to_f64(O.normal(63, (nq, D), 0.0, 1.0, BF16), BF16)) + 0.25
+    K = O.to_f64(O.normal(64, (keys, nkv, D), 0.0, 1.0, BF16), BF16)
+    V = O.to_f64(O.normal(65, (keys, nkv, D), 0.0, 1.0, BF16), BF16)
+    q = O.to_f64(O.from_f64(q, BF16), BF16)
+
+    def run(Kx):
+        dev = (to_dev(O.from_f64(t, BF16), BF16) for t in (q, Kx, V))
+        return prims.attn_decode(*dev, keys - 1, 0.088).cpu().numpy().astype(np.float64)
+
+    base = run(K)
+    assert np.isfinite(base).all()
+    bad = K.copy()
+    bad[-1, 3, 5] = np.nan
+    out = run(bad)
+    assert np.isnan(out[15:20]).all()
+    assert np.array_equal(np.delete(out, range(15, 20), 0), np.delete(base, range(15, 20), 0))
+    if keys > 40:
+        low = K.copy()
+        low[-1, 3, 5] = -np.inf   # q > 0: a score of -inf
+        low[:32, 6, 9] = -np.inf
+        out = run(low)
+        s32 = float(np.float32(0.088))
+        for h in range(nq):
+            g = h // 5
+            live = np.isfinite(low[:, g]).all(-1)
+            s = (low[live, g] @ q[h]) * s32
+            p = np.exp(s - s.max())
+            p /= p.sum()
+            assert np.all(np.abs(out[h] - p @ V[live, g]) <= 5e-5 * (p @ np.abs(V[live, g]))), h
