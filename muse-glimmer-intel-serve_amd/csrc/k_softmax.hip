@@ -382,8 +382,12 @@ namespace mg
 
     // those scores to 2^(s c2 - mc); returns the wave's sum. mc = the maximum
     // times c2, rounded, and 0 where the maximum is -inf: -inf scores then weigh
-    // 0 and a NaN one, which no maximum shows, still reaches the sum
-    template <int CH, int WPR>
+    // 0 and a NaN one, which no maximum shows, still reaches the sum. A weight at
+    // the maximum is 2^(mc's rounding error), the same factor in every weight and
+    // the sum: it cancels while |mc| is below kFastMax (2^+-2 there). FAR: mc is
+    // the maximum itself, and the weights are 2^((s - mc) c2), of any magnitude.
+    constexpr float kFastMax = 0x1p26f;
+    template <int CH, int WPR, bool FAR>
     MG_DEV float fast_exp(float c2, float mc, int w, FastRow<CH> &r)
     {
         const int lo = int(r.lo64), hi = int(r.hi64);
@@ -394,7 +398,7 @@ namespace mg
             if (cb > hi || cb + 511 < lo) continue;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                r.v[c][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(r.v[c][e], c2, -mc));
+                r.v[c][e] = __builtin_amdgcn_exp2f(FAR ? (r.v[c][e] - mc) * c2 : __builtin_fmaf(r.v[c][e], c2, -mc));
                 sum += r.v[c][e];
             }
         }
@@ -451,10 +455,12 @@ namespace mg
         if (!r.live) return;
         __shared__ double tab[CAP ? 128 : 1];
         const float m = fast_scores<CH, 1, CAP>(a, lane, 0, r, tab);
-        const float sum = fast_exp<CH, 1>(c2, m == kNegInf ? 0.0f : m * c2, 0, r);
-        // a row with non-finite sums is redone on the accurate path (NaN scores only:
-        // the maximum is -inf, the sum NaN)
-        if (!(sum < __builtin_huge_valf())) {
+        const float mc = m == kNegInf ? 0.0f : m * c2;
+        const float sum = fast_exp<CH, 1, false>(c2, mc, 0, r);
+        // redone on the accurate path: a row with a NaN sum (NaN scores only: the
+        // maximum is -inf, the sum NaN) and one whose maximum lies past kFastMax,
+        // where the rounding of mc no longer cancels within f32's range
+        if (!(sum < __builtin_huge_valf()) || !(__builtin_fabsf(mc) < kFastMax)) {
             softmax_row_accurate<SF32, SO, CH, CAP>(a, x + row * a.ldx, y + row * a.ldy, r.lo64, r.hi64, VEC, lane);
             return;
         }
@@ -487,7 +493,7 @@ namespace mg
         float M = red[0];
 #pragma unroll
         for (int i = 1; i < WPR; ++i) M = __builtin_fmaxf(M, red[i]);
-        const float sum = fast_exp<CH, WPR>(c2, M == kNegInf ? 0.0f : M * c2, w, r);
+        const float sum = fast_exp<CH, WPR, true>(c2, M == kNegInf ? 0.0f : M, w, r);
         if (lane == 0) red[WPR + w] = sum;
         __syncthreads();
         float L = 0.0f;

@@ -410,3 +410,22 @@ def test_split_rows_of_nan(prims, dt_in, dt_out, kc, softcap):
     assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.isnan(ref[0, :3]).any(-1).all()
     ok = ~np.isnan(ref) & (ref > 1e-30)
     assert np.abs(y[ok] / ref[ok] - 1.0).max() < 2.0 ** -7
+
+
+@pytest.mark.parametrize("kc", (512, 2048, 2049, 4100, 8200))
+@pytest.mark.parametrize("dt_out", (BF16, F16))
+def test_scores_of_any_magnitude(prims, kc, dt_out):
+    """finite scores past 2^26 in the log2 domain: rows of the type's lowest value
+    only and of 1e12 only (every visible key the same weight), lowest values beside
+    ordinary scores, and ordinary differences about a large common value"""
+    low = np.finfo(np.float32).min
+    x = O.to_f64(O.normal(20, (1, 8, kc), 0.0, 3.0, F32), F32).astype(np.float32)
+    x[0, 0, :] = low
+    x[0, 1, :] = 1e12
+    x[0, 2, 1::2] = low
+    x[0, 3, : kc - 20] = low                 # a whole wave's keys and more
+    x[0, 4] += np.float32(2.0 ** 32)         # multiples of 512: scores 45 apart
+    x[0, 5] += np.float32(-2.0 ** 34)
+    x[0, 6, 0] = -low                        # one key takes all
+    y, ref = scores_case(prims, x, kc - 8, dt_out=dt_out)
+    assert np.all(ulp_diff16(y, ref) <= 1), [int(ulp_diff16(y[0, r], ref[0, r]).max()) for r in range(8)]
