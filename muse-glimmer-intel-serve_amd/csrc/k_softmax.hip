@@ -380,29 +380,70 @@ namespace mg
         return dpp_max(m);
     }
 
-    // those scores to 2^(s c2 - mc); returns the wave's sum. mc = the maximum
-    // times c2, rounded, and 0 where the maximum is -inf: -inf scores then weigh
-    // 0 and a NaN one, which no maximum shows, still reaches the sum. A weight at
-    // the maximum is 2^(mc's rounding error), the same factor in every weight and
-    // the sum: it cancels while |mc| is below kFastMax (2^+-2 there). FAR: mc is
-    // the maximum itself, and the weights are 2^((s - mc) c2), of any magnitude.
+    // one wave's row: those scores to 2^(s c2 - mc); returns their sum. mc = the
+    // maximum times c2, rounded, and 0 where the maximum is -inf: -inf scores then
+    // weigh 0 and a NaN one, which no maximum shows, still reaches the sum. A weight
+    // at the maximum is 2^(mc's rounding error), the same factor in every weight and
+    // the sum: it cancels while |mc| is below kFastMax (2^+-2 there).
     constexpr float kFastMax = 0x1p26f;
-    template <int CH, int WPR, bool FAR>
-    MG_DEV float fast_exp(float c2, float mc, int w, FastRow<CH> &r)
+    template <int CH>
+    MG_DEV float fast_exp(float c2, float mc, FastRow<CH> &r)
     {
         const int lo = int(r.lo64), hi = int(r.hi64);
         float sum = 0.0f;
 #pragma unroll
         for (int c = 0; c < CH; ++c) {
-            const int cb = (c * WPR + w) * 512;
+            const int cb = c * 512;
             if (cb > hi || cb + 511 < lo) continue;
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                r.v[c][e] = __builtin_amdgcn_exp2f(FAR ? (r.v[c][e] - mc) * c2 : __builtin_fmaf(r.v[c][e], c2, -mc));
+                r.v[c][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(r.v[c][e], c2, -mc));
                 sum += r.v[c][e];
             }
         }
         return dpp_sum_f32(sum);
+    }
+
+    // a work-group's row: the wave's scores to their weights relative to the row's
+    // maximum M (0 for -inf), returning the wave's sum; precision as in the split
+    // passes below. Without a cap 2^(s c2 - mc), 2^((s - M) c2) where |mc| reaches
+    // kFastMax, eight of a lane summed in f32 and the rest in f64; with one the
+    // accurate exponential of the exact difference, summed in f64. (Hardware exp2 and
+    // f32 sums took 82 us instead of 105 for 16000 capped rows of 4000, and missed the
+    // nearest bf16 for 1.68e-4 of the probabilities instead of 1.39e-4, the split
+    // passes 1.38e-4; without a cap f64 costs nothing and 7.8e-6 become 5.6e-6.)
+    template <int CH, int WPR, bool CAP>
+    MG_DEV double group_exp(float c2, float M, int w, FastRow<CH> &r)
+    {
+        const int lo = int(r.lo64), hi = int(r.hi64);
+        const float mc = M * c2;
+        const bool far = !CAP && !(__builtin_fabsf(mc) < kFastMax);
+        double sum = 0.0;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const int cb = (c * WPR + w) * 512;
+            if (cb > hi || cb + 511 < lo) continue;
+            if constexpr (CAP) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    r.v[c][e] = r.v[c][e] == kNegInf ? 0.0f : exp_diff(r.v[c][e], M);
+                    sum += double(r.v[c][e]);
+                }
+            } else {
+                if (far) { // (uniform)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) r.v[c][e] = __builtin_amdgcn_exp2f((r.v[c][e] - M) * c2);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) r.v[c][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(r.v[c][e], c2, -mc));
+                }
+                float part = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) part += r.v[c][e];
+                sum += double(part);
+            }
+        }
+        return dpp_sum(sum);
     }
 
     // the wave's share of the row times `f` to storage; chunks without a visible
@@ -456,7 +497,7 @@ namespace mg
         __shared__ double tab[CAP ? 128 : 1];
         const float m = fast_scores<CH, 1, CAP>(a, lane, 0, r, tab);
         const float mc = m == kNegInf ? 0.0f : m * c2;
-        const float sum = fast_exp<CH, 1, false>(c2, mc, 0, r);
+        const float sum = fast_exp<CH>(c2, mc, r);
         // redone on the accurate path: a row with a NaN sum (NaN scores only: the
         // maximum is -inf, the sum NaN) and one whose maximum lies past kFastMax,
         // where the rounding of mc no longer cancels within f32's range
@@ -481,7 +522,8 @@ namespace mg
     {
         using ro = typename SO::raw;
         constexpr int CH = 4;
-        __shared__ float red[2 * WPR];
+        __shared__ float red[WPR];
+        __shared__ double redd[WPR];
         const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
         const int64_t row = blockIdx.x;
         FastRow<CH> r;
@@ -493,19 +535,19 @@ namespace mg
         float M = red[0];
 #pragma unroll
         for (int i = 1; i < WPR; ++i) M = __builtin_fmaxf(M, red[i]);
-        const float sum = fast_exp<CH, WPR, true>(c2, M == kNegInf ? 0.0f : M, w, r);
-        if (lane == 0) red[WPR + w] = sum;
+        const double sum = group_exp<CH, WPR, CAP>(c2, M == kNegInf ? 0.0f : M, w, r);
+        if (lane == 0) redd[w] = sum;
         __syncthreads();
-        float L = 0.0f;
+        double L = 0.0;
 #pragma unroll
-        for (int i = 0; i < WPR; ++i) L += red[WPR + i];
-        if (!(L < __builtin_huge_valf())) {
+        for (int i = 0; i < WPR; ++i) L += redd[i];
+        if (L != L) {
             ro *yr = y + row * a.ldy;
             for (int j = int(threadIdx.x); j < int(a.kc); j += 64 * WPR)
                 yr[j] = j >= int(r.lo64) && j <= int(r.hi64) ? SO::enc32(__builtin_nanf("")) : ro(0);
             return;
         }
-        fast_store<SO, CH, WPR, VEC>(a, y, row, __builtin_amdgcn_rcpf(L), M == kNegInf, lane, w, r);
+        fast_store<SO, CH, WPR, VEC>(a, y, row, float(1.0 / L), M == kNegInf, lane, w, r);
     }
 
     // ------------------------------------------------------------- split rows
