@@ -65,42 +65,65 @@ namespace mg
         return s;
     }
 
-    // the plain capped-score chain for the keys the fast one does not certify;
-    // out of line, so the unrolled per-key code stays small
-    __attribute__((noinline)) __device__ float capped_score_slow(float x, float scale, float cap)
-    {
-        const float s = (x * scale) / cap; // f32 operations: the twin's f64 ones rounded to f32
-        return float(mgm::tanh(double(s))) * cap;
-    }
-
     // the tanh table's copy in a wave's own LDS, made when its first key needs it
+    typedef const double __attribute__((address_space(3))) *LdsTab;
     struct CapTab
     {
         double *tab; // 128 entries
         bool have;
     };
 
+    // The two functions below are out of line: the unrolled per-key code stays small,
+    // and the kernels' registers are their own.
+    // The plain capped-score chain, f32 operations with the twin's f64 tanh between.
+    __attribute__((noinline)) __device__ float capped_score_plain(float x, float scale, float cap)
+    {
+        return float(mgm::tanh(double((x * scale) / cap))) * cap;
+    }
+    // The capped scores of two keys with a bit set in `need` (their v is the raw score,
+    // the others' stays) by the tail's table polynomial, where both ends of its error
+    // interval round to one f32 (tests/test_tanh_fast.py runs every f32 below 22); the
+    // bits of those where they do not stay in `need`.
+    struct CapKeys
+    {
+        float v[2];
+        uint32_t need;
+    };
+    __attribute__((noinline)) __device__ CapKeys capped_score_table(CapKeys k, float scale, float cap, float rcap, LdsTab tab)
+    {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const float s = k.v[i] * scale, as = __builtin_fabsf(s);
+            const float q = mgm::softcap_quotient(s, cap, rcap);
+            const double aq = __builtin_fabs(double(q)), a = __builtin_fmin(aq, 0x1.fffffffffffffp-1);
+            double tl, tu;
+            mgm::tanh_interval(mgm::tanh_table_at(a, tab[int(a * 128.0)]), tl, tu);
+            const float lo = float(tl);
+            const bool take = ((k.need >> i) & 1u) && as > 0x1p-100f && as < 0x1p100f && aq < 1.0 && lo == float(tu);
+            k.v[i] = take ? __builtin_copysignf(lo, q) * cap : k.v[i];
+            k.need &= take ? ~(1u << i) : ~0u;
+        }
+        return k;
+    }
+
     // 8 raw f32 scores of a row -> capped scores (bit e of vis set: key e is
-    // visible, else it becomes -inf). Each key takes mgm::softcap_score_fast.
-    // A wave with a key it does not certify (|s / cap| >= 2^-5, or a rounding
-    // too close to call) evaluates the tail's table polynomial for its keys, four
-    // side by side without a branch, and takes it where both ends of its error
-    // interval round to one f32 (tests/test_tanh_fast.py runs every f32 below 22);
-    // the rest (|s / cap| >= 1, inf, NaN, about 3 in 10^6 others) are redone by
-    // the plain chain. Bits are the twin's on every path. Scores of std 5 under
-    // a cap of 30 (most of them past 2^-5), [40, 2048, 2048]: 419 -> 219 us against
-    // the plain chain in the table's place.
+    // visible, else it becomes -inf). Each key takes mgm::softcap_score_fast. Where
+    // that certifies not every lane's (|s / cap| >= 2^-5, or a rounding too close to
+    // call) two key slots at a time go to capped_score_table: scores of std 3 under a
+    // cap of 30 leave 6 in 100 pairs of slots to it. Bits are the twin's on every path.
+    // [40, 2048, 2048], cap 30: 117 us at std 3 (89 registers, five waves a SIMD),
+    // 215 at std 20 and more. All eight keys in line, four side by side: 135 and 211
+    // (four waves); one key a call: 119 and 212, rows too few to fill the chip 1.15 of
+    // the time; the plain chain alone in the table's place 116 and 350 to 418.
     MG_DEV void cap8(const SmArgs &a, float *v, uint32_t vis, CapTab &ct)
     {
-        float x[8];
-        uint32_t slow = 0;
+        uint32_t slow = 0; // keys whose v is still the raw score
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            x[e] = v[e];
             bool ok;
-            const float c = mgm::softcap_score_fast(x[e], a.scale, a.cap, a.rcap, ok);
+            const float c = mgm::softcap_score_fast(v[e], a.scale, a.cap, a.rcap, ok);
             const bool in = (vis >> e) & 1u;
-            v[e] = in ? c : kNegInf;
+            v[e] = !in ? kNegInf : ok ? c : v[e];
             slow |= uint32_t(in && !ok) << e;
         }
         if (__builtin_amdgcn_ballot_w64(slow != 0u)) {
@@ -111,26 +134,20 @@ namespace mg
                 wave_lds_sync();
                 ct.have = true;
             }
+            uint32_t left = 0;
 #pragma unroll
-            for (int g = 0; g < 8; g += 4) {
+            for (int e = 0; e < 8; e += 2)
+                if (__builtin_amdgcn_ballot_w64(((slow >> e) & 3u) != 0u)) {
+                    const CapKeys k = capped_score_table({{v[e], v[e + 1]}, slow >> e}, a.scale, a.cap, a.rcap, (LdsTab)ct.tab);
 #pragma unroll
-                for (int e = g; e < g + 4; ++e) {
-                    const float s = x[e] * a.scale, as = __builtin_fabsf(s);
-                    const float q = mgm::softcap_quotient(s, a.cap, a.rcap);
-                    const double aq = __builtin_fabs(double(q));
-                    double tl, tu;
-                    mgm::tanh_interval(mgm::tanh_table_abs(__builtin_fmin(aq, 0x1.fffffffffffffp-1), ct.tab), tl, tu);
-                    const float lo = float(tl);
-                    const bool ok = as > 0x1p-100f && as < 0x1p100f && aq < 1.0 && lo == float(tu);
-                    const bool take = ok && ((slow >> e) & 1u);
-                    v[e] = take ? __builtin_copysignf(lo, q) * a.cap : v[e];
-                    slow &= take ? ~(1u << e) : ~0u;
+                    for (int i = 0; i < 2; ++i) v[e + i] = k.v[i];
+                    left |= (k.need & 3u) << e;
                 }
-            }
-            if (__builtin_amdgcn_ballot_w64(slow != 0u)) {
+            // |s / cap| >= 1, inf, NaN, and about 3 in 10^5 others
+            if (__builtin_amdgcn_ballot_w64(left != 0u)) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    if ((slow >> e) & 1u) v[e] = capped_score_slow(x[e], a.scale, a.cap);
+                    if ((left >> e) & 1u) v[e] = capped_score_plain(v[e], a.scale, a.cap);
             }
         }
     }
@@ -483,6 +500,41 @@ namespace mg
         }
     }
 
+    // a row with NaN among its visible scores, or +inf without a cap: NaN at the
+    // visible keys, 0 at the others
+    template <class SO>
+    MG_DEV void store_nan_row(typename SO::raw *yr, int lo, int hi, int kc, int tid, int threads)
+    {
+#pragma unroll 1
+        for (int j = tid; j < kc; j += threads) yr[j] = SO::enc32(j >= lo && j <= hi ? __builtin_nanf("") : 0.0f);
+    }
+
+    // A row of scores that the one-wave kernel hands back, by the accurate row's
+    // arithmetic, read three times key by key: rare, and out of line so that its
+    // registers are not the kernel's (with the accurate row inlined k_softmax_fast<4>
+    // took 105 to 119; 96 allow five waves a SIMD)
+    template <class SO>
+    __attribute__((noinline)) __device__ void softmax_row_redo(const float *xr, typename SO::raw *yr, float scale, int lo,
+                                                               int hi, int kc, int lane)
+    {
+        float m = kNegInf;
+#pragma unroll 1
+        for (int j = lo + lane; j <= hi; j += 64) m = __builtin_fmaxf(m, xr[j] * scale);
+        m = dpp_max(m);
+        auto weight = [&](float s) { return s == kNegInf ? 0.0f : exp_diff(s, m); };
+        double sum = 0.0;
+#pragma unroll 1
+        for (int j = lo + lane; j <= hi; j += 64) sum += double(weight(xr[j] * scale));
+        sum = dpp_sum(sum);
+        if (sum != sum) {
+            store_nan_row<SO>(yr, lo, hi, kc, lane, 64);
+            return;
+        }
+        const float inv = sum == 0.0 ? 0.0f : float(1.0 / sum);
+#pragma unroll 1
+        for (int j = lane; j < kc; j += 64) yr[j] = SO::enc32(j < lo || j > hi ? 0.0f : weight(xr[j] * scale) * inv);
+    }
+
     // One row per one-wave work-group. All of the row's loads are issued
     // before the first is used, and the compiler waits for each chunk's own.
     template <class SO, int CH, bool CAP, bool VEC>
@@ -498,11 +550,16 @@ namespace mg
         const float m = fast_scores<CH, 1, CAP>(a, lane, 0, r, tab);
         const float mc = m == kNegInf ? 0.0f : m * c2;
         const float sum = fast_exp<CH>(c2, mc, r);
-        // redone on the accurate path: a row with a NaN sum (NaN scores only: the
-        // maximum is -inf, the sum NaN) and one whose maximum lies past kFastMax,
-        // where the rounding of mc no longer cancels within f32's range
-        if (!(sum < __builtin_huge_valf()) || !(__builtin_fabsf(mc) < kFastMax)) {
-            softmax_row_accurate<SF32, SO, CH, CAP>(a, x + row * a.ldx, y + row * a.ldy, r.lo64, r.hi64, VEC, lane);
+        // a NaN sum (NaN scores only: the maximum is -inf, the sum NaN), or a maximum
+        // past kFastMax, where the rounding of mc no longer cancels within f32's
+        // range (capped scores stay below it)
+        const bool nan = !(sum < __builtin_huge_valf());
+        if (CAP && nan) {
+            store_nan_row<SO>(y + row * a.ldy, int(r.lo64), int(r.hi64), int(a.kc), lane, 64);
+            return;
+        }
+        if (!CAP && (nan || !(__builtin_fabsf(mc) < kFastMax))) {
+            softmax_row_redo<SO>(x + row * a.ldx, y + row * a.ldy, a.scale, int(r.lo64), int(r.hi64), int(a.kc), lane);
             return;
         }
         fast_store<SO, CH, 1, VEC>(a, y, row, m == kNegInf ? 0.0f : __builtin_amdgcn_rcpf(sum), m == kNegInf, lane, 0, r);
@@ -520,7 +577,6 @@ namespace mg
     __global__ __launch_bounds__(64 * WPR) void k_softmax_group(const float *__restrict__ x,
                                                                 typename SO::raw *__restrict__ y, SmArgs a, float c2)
     {
-        using ro = typename SO::raw;
         constexpr int CH = 4;
         __shared__ float red[WPR];
         __shared__ double redd[WPR];
@@ -542,9 +598,7 @@ namespace mg
 #pragma unroll
         for (int i = 0; i < WPR; ++i) L += redd[i];
         if (L != L) {
-            ro *yr = y + row * a.ldy;
-            for (int j = int(threadIdx.x); j < int(a.kc); j += 64 * WPR)
-                yr[j] = j >= int(r.lo64) && j <= int(r.hi64) ? SO::enc32(__builtin_nanf("")) : ro(0);
+            store_nan_row<SO>(y + row * a.ldy, int(r.lo64), int(r.hi64), int(a.kc), int(threadIdx.x), 64 * WPR);
             return;
         }
         fast_store<SO, CH, WPR, VEC>(a, y, row, float(1.0 / L), M == kNegInf, lane, w, r);

@@ -80,11 +80,11 @@ namespace mgm
     // the branch of tanh_fast_abs for 0 <= a < 1 (d = a - a0 is exact):
     //   tanh(a0 + d) = t0 + (1 - t0^2) d [1 - t0 d + (t0^2 - 1/3) d^2
     //                  + t0 (2/3 - t0^2) d^3 + (2/15 - t0^2 + t0^4) d^4] + R
-    // (tab: kTanhTab or a copy of it, e.g. in a work-group's shared memory)
-    MG_TF double tanh_table_abs(double a, const double *tab = kTanhTab)
+    // (t: the table's entry int(a * 128))
+    MG_TF double tanh_table_at(double a, double t)
     {
         const int k = int(a * 128.0);
-        const double t = tab[k], u = t * t;
+        const double u = t * t;
         const double d = a - (k == 0 ? 0.0 : (double(k) + 0.5) * 0x1p-7); // interval 0: about 0
         double e = __builtin_fma(u, u - 1.0, 2.0 / 15.0);
         e = __builtin_fma(d, e, t * (2.0 / 3.0 - u));
@@ -93,6 +93,9 @@ namespace mgm
         e = __builtin_fma(d, e, 1.0);
         return __builtin_fma((1.0 - u) * d, e, t);
     }
+
+    // (tab: kTanhTab or a copy of it, e.g. in a work-group's shared memory)
+    MG_TF double tanh_table_abs(double a, const double *tab = kTanhTab) { return tanh_table_at(a, tab[int(a * 128.0)]); }
 
     // the interval t (1 -+ m) that a caller rounds at both ends, one rounding each
     MG_TF void tanh_interval(double t, double &lo, double &hi, double m = kTanhFastMargin)
