@@ -412,11 +412,21 @@ namespace mg
         need(aligned16(qs) && aligned16(x) && ldx % 8 == 0, "gemv_q8_0: quants and activations must be 16-byte aligned");
         if (rows == 0) return;
         need(rows < (int64_t(1) << 33), "gemv_q8_0: too many rows");
-        // rows of whole 256-quant pieces: the matrix cores from two activation rows
-        // on (one row: 34-36 us against the vector form's 26 at [25600, 5120]); two
-        // rows only over a weight of 2^26 quants and more (10.4 us against 9.4 at
-        // [5120, 5120], 32-34 against 35 at [25600, 5120], 31 against 41 at [6656, 19968])
-        if ((batch > 2 || (batch == 2 && rows * in >= (int64_t(1) << 26))) && !blockdot && in % 256 == 0 && in > 0 && aligned16(d)) {
+        // rows of whole 256-quant pieces: the matrix cores where they are the faster
+        // form. Five activation rows and more take the weights twice in the vector
+        // form, and it loses everywhere ([256, 5120] 6.2 us against 6.9, but in a second
+        // launch). Fewer rows on a small weight leave the matrix form's 16
+        // rows a work-group too few work-groups, so the line lies, vector against matrix
+        // form (kernel times, in a graph):
+        //   4 rows  [2048, 8192] 10.2 / 10.7, [3000, 16384] 21.7 / 18.9, [1024, 5120] 3.9 / 7.0
+        //   3 rows  [3000, 16384] 16.6 / 18.7, [5120, 5120] 10.3 / 10.6, [5120, 8192] 15.9 / 14.5
+        //   2 rows  [5120, 8192] 13.4 / 14.6, [8192, 10240] 24.4 / 18.5, [5120, 25600]
+        //           39.6 / 37.9; short weight rows later: [20000, 4096] 20.6 / 21.3,
+        //           [28672, 4096] 28.8 / 26.9
+        // (one row: 26 / 34 to 36 at [25600, 5120])
+        const bool matrix = batch >= 5 || (batch == 4 && rows > 2048) || (batch == 3 && rows >= 4096 && rows * in >= (int64_t(1) << 25)) ||
+                            (batch == 2 && rows >= 5120 && rows * in >= (in >= 5120 ? int64_t(1) << 26 : int64_t(100000000)));
+        if (matrix && !blockdot && in % 256 == 0 && in > 0 && aligned16(d)) {
             auto go = [&](auto kern, int64_t rt, int waves) {
                 hipLaunchKernelGGL(kern, dim3(unsigned((rows + 16 * rt - 1) / (16 * rt))), dim3(unsigned(64 * waves)), 0,
                                    c->stream, qs, d, x, y, in, rows, ldx, ldy, int(batch));

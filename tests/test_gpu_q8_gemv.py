@@ -101,18 +101,42 @@ def test_gemv_widths(prims, n_in, blockdot):
 
 
 @pytest.mark.parametrize("rows,n_in,B", ((1, 256, 2), (15, 512, 8), (17, 1280, 3), (33, 2304, 7), (4111, 256, 6),
-                                         (4127, 2304, 5), (16390, 512, 8)))
+                                         (4127, 2304, 5), (16390, 512, 8),
+                                         (2048, 256, 4), (2049, 1280, 4)))
 def test_gemv_matrix_cores(prims, rows, n_in, B):
-    """two to eight activation rows over rows of whole 256-quant pieces: tiles of
-    16 and 32 weight rows with remainders, fewer pieces than waves, uneven pieces"""
+    """activation rows over rows of whole 256-quant pieces: tiles of 16 and 32 weight
+    rows with remainders, fewer pieces than waves, uneven pieces, and both sides of
+    the line for four rows (few weight rows and two or three activation rows take
+    the vector form)"""
     gemv_case(prims, rows, n_in, B, False)
 
 
-def test_gemv_matrix_cores_strides_and_nonfinite(prims):
-    """strided activations and outputs; an infinite and a NaN activation row and
+@pytest.mark.parametrize("rows,n_in,B", ((5119, 13312, 2), (5125, 13312, 2), (24500, 4096, 2), (4095, 8448, 3),
+                                         (4097, 8192, 3), (4111, 8448, 3)))
+def test_gemv_two_and_three_rows(prims, rows, n_in, B):
+    """two and three activation rows on both sides of their lines (weights from 2^25
+    and 2^26 quants): against the f64 sum of the same terms on the device"""
+    import torch
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(rows)
+    qs = torch.randint(-127, 128, (rows, n_in), generator=g, dtype=torch.int8, device="cuda:0")
+    d = (torch.rand((rows, n_in // 32), generator=g, device="cuda:0") * 2e-2 + 1e-3).half()
+    x = torch.randn((B, n_in), generator=g, device="cuda:0").bfloat16()
+    y = torch.empty((B, rows), device="cuda:0")
+    prims.gemv_q8_0(qs, d, x, y)
+    for r in range(0, rows, 2048):
+        w = (qs[r:r + 2048].float() * d[r:r + 2048].float().repeat_interleave(32, 1)).bfloat16().double().t().contiguous()
+        err = (y[:, r:r + 2048].double() - x.double() @ w).abs()
+        assert torch.all(err <= 1e-5 * (x.double().abs() @ w.abs()))
+
+
+@pytest.mark.parametrize("rows", (40, 2060))
+def test_gemv_matrix_cores_strides_and_nonfinite(prims, rows):
+    """(2060 weight rows on the matrix cores, 40 in the vector form)
+    strided activations and outputs; an infinite and a NaN activation row and
     a weight row with an infinite scale reach only their own outputs"""
     import torch
-    rows, n_in, B = 40, 512, 4
+    n_in, B = 512, 4
     qs = torch.randint(-127, 128, (rows, n_in), dtype=torch.int8, device="cuda:0")
     d = torch.full((rows, n_in // 32), 0.01, dtype=torch.float16, device="cuda:0")
     d[7, 3] = float("inf")
