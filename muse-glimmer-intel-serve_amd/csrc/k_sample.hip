@@ -15,6 +15,8 @@
 #include "mg_internal.hpp"
 #include "mg_wave_sort.hpp"
 
+#include <cmath>
+
 namespace mg
 {
     MG_DEV double wave_incl_scan(double v)
@@ -1205,6 +1207,7 @@ namespace mg
         SliceStat *stat; // [rows][G]
         uint64_t *keys;  // [rows][G][M]
         int M;
+        int lane_rank, wave_rank; // T0 (slice_ranks)
     };
     struct SfSliceLds : SfRed
     {
@@ -1218,9 +1221,29 @@ namespace mg
         int len[2][kSliceMax];
     };
 
-    // kRank: for NV * 4 random entries a thread, about 0.8 M keys lie at or above the
-    // kRank-th largest of 64 thread maxima (M = 1024 at NV 7, 512 at NV 4)
-    template <int NV, int kRank>
+    // T0's ranks: the lane_rank-th largest thread maximum of each wave, the
+    // wave_rank-th largest of those. A slice holds V / G of the row's entries in KiB
+    // chunks, dealt to its 16 waves in turn (fewer of them where it has fewer chunks):
+    // m entries a lane of the waves that hold some. About 0.8 M random keys reach T0
+    // where a share 1 - (1 - p)^m of the lanes has one of them, p = 0.8 M G / V, and
+    // the middle wave stands for them all. (Simulated for V from 16384 to 458752: 0.73
+    // to 0.89 M keys, above M in one slice of 60 at most, and never fewer than 4096 of
+    // the row's keys above every slice's end. Ranks fitted to one V left runs half
+    // empty at others, and every row to the one-work-group algorithm: 64 rows of
+    // 128256, a nucleus of 4096 and more, 73 us before there were slices, 156 with the
+    // fitted ranks, 56 now.)
+    inline void slice_ranks(int64_t V, int G, SliceWork &w)
+    {
+        const int64_t chunks = (V + 255) / 256;
+        const int waves = int(chunks / G < 16 ? chunks / G : 16);
+        const double m = double(V) / G / (64.0 * waves), p = 0.8 * double(w.M) * G / double(V);
+        const double share = p < 1.0 ? 1.0 - std::pow(1.0 - p, m) : 1.0;
+        const int k = int(std::lrint(64.0 * share));
+        w.lane_rank = k < 1 ? 1 : k > 64 ? 64 : k;
+        w.wave_rank = (waves + 1) / 2;
+    }
+
+    template <int NV>
     __global__ __launch_bounds__(kSfThreads) void k_sample_slice(const float *__restrict__ lg, int64_t ld, int64_t V,
                                                                 float temperature, SliceWork w)
     {
@@ -1252,14 +1275,14 @@ namespace mg
                 nc += sf_cand(x[i][e]) ? 1u : 0u;
                 nfin += __builtin_isfinite(x[i][e]) ? 1u : 0u;
             }
-        // the slice's counts and maximum, and T0: each wave's kRank-th largest thread
+        // the slice's counts and maximum, and T0: each wave's lane_rank-th largest thread
         // maximum, the eighth largest of those over the waves
         const uint64_t cnt = sf_sum_u64((uint64_t(nc) << 32) | nfin, L);
         nc = uint32_t(cnt >> 32);
         nfin = uint32_t(cnt);
         uint32_t im[1] = {f32_key(m1 + 0.0f)};
         wave_bitonic_desc<uint32_t, 1>(im);
-        if (lane == 0) L.redu[wv] = (uint64_t(im[0]) << 32) | uint32_t(__builtin_amdgcn_readlane(int(im[0]), kRank - 1));
+        if (lane == 0) L.redu[wv] = (uint64_t(im[0]) << 32) | uint32_t(__builtin_amdgcn_readlane(int(im[0]), w.lane_rank - 1));
         __syncthreads();
         const uint64_t wm = L.redu[lane & 15];
         const uint32_t big = dpp_max_u32(uint32_t(wm >> 32)), mid = uint32_t(wm);
@@ -1269,7 +1292,7 @@ namespace mg
             const uint32_t o = uint32_t(__builtin_amdgcn_readlane(int(mid), i));
             above += o > mid || (o == mid && i < (lane & 15)) ? 1 : 0;
         }
-        const uint32_t t0 = uint32_t(__builtin_amdgcn_readlane(int(mid), int(__builtin_ctzll(__builtin_amdgcn_ballot_w64(above == 7)))));
+        const uint32_t t0 = uint32_t(__builtin_amdgcn_readlane(int(mid), int(__builtin_ctzll(__builtin_amdgcn_ballot_w64(above == w.wave_rank - 1)))));
         const float mx = key_f32(big);
         float T0 = key_f32(t0);
         __syncthreads();
@@ -1571,21 +1594,26 @@ namespace mg
         auto vecs = [&](int G) { return ((V + 3) / 4 + int64_t(kSfThreads) * G - 1) / (int64_t(kSfThreads) * G); };
         int GS = rows <= 16 ? 16 : 8;
         while (GS < kSliceMax && vecs(GS) > kSliceVec) GS *= 2;
+        // (one work-group a CU past 4 vectors, two rounds of them at most; past 262144
+        // entries also below: 64 rows of 300000 in 1024 work-groups 128 us, the split
+        // path 95)
+        const bool few = rows * GS <= 512 || V <= 262144;
         const int64_t b_slice = (rows * GS * int64_t(sizeof(SliceStat)) + 255) / 256 * 256;
-        if (sorted && (top_k <= 0 || top_k >= V) && rows <= 64 && V >= 4 * 4096 && vecs(GS) <= kSliceVec &&
+        if (sorted && (top_k <= 0 || top_k >= V) && rows <= 64 && few && V >= 4 * 4096 && vecs(GS) <= kSliceVec &&
             b_slice + rows * kSliceKeys * 8 <= c->work_bytes) {
             SliceWork sw;
             sw.stat = static_cast<SliceStat *>(c->work);
             sw.keys = reinterpret_cast<uint64_t *>(static_cast<char *>(c->work) + b_slice);
             sw.M = kSliceKeys / GS;
+            slice_ranks(V, GS, sw);
             auto go = [&](auto kern) {
                 hipLaunchKernelGGL(kern, dim3(unsigned(GS), unsigned(rows)), dim3(kSfThreads), 0, c->stream, lg, ld, V, T, sw);
             };
             const int64_t nv = vecs(GS);
             if (nv <= 4)
-                go(k_sample_slice<4, 21>);
+                go(k_sample_slice<4>);
             else
-                go(k_sample_slice<kSliceVec, 35>);
+                go(k_sample_slice<kSliceVec>);
             check_launch("k_sample_slice");
             hipLaunchKernelGGL(k_sample_finish, dim3(unsigned(rows)), dim3(kSfThreads), 0, c->stream, lg, ld, V,
                                raw_amax, top_k, GS, T, tp, mp, out_ids, out_p, out_n, sw);
