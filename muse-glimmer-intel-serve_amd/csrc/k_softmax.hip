@@ -246,6 +246,13 @@ namespace mg
 #pragma unroll
         for (int e = 0; e < 8; ++e) p[e] = j0 + e >= lo && j0 + e <= hi ? __builtin_nanf("") : 0.0f;
     }
+    // the same to keys j, j + threads, ... below `end` of the row
+    template <class SO>
+    MG_DEV void store_nan_row(typename SO::raw *yr, int64_t lo, int64_t hi, int64_t j, int64_t end, int threads)
+    {
+#pragma unroll 1
+        for (; j < end; j += threads) yr[j] = SO::enc32(j >= lo && j <= hi ? __builtin_nanf("") : 0.0f);
+    }
 
     // --------------------------------------------------------- one wave per row
     // Accurate row: transformed scores, exp of the exactly formed s - max, f64
@@ -500,15 +507,6 @@ namespace mg
         }
     }
 
-    // a row with NaN among its visible scores, or +inf without a cap: NaN at the
-    // visible keys, 0 at the others
-    template <class SO>
-    MG_DEV void store_nan_row(typename SO::raw *yr, int lo, int hi, int kc, int tid, int threads)
-    {
-#pragma unroll 1
-        for (int j = tid; j < kc; j += threads) yr[j] = SO::enc32(j >= lo && j <= hi ? __builtin_nanf("") : 0.0f);
-    }
-
     // A row of scores that the one-wave kernel hands back, by the accurate row's
     // arithmetic, read three times key by key: rare, and out of line so that its
     // registers are not the kernel's (with the accurate row inlined k_softmax_fast<4>
@@ -527,7 +525,7 @@ namespace mg
         for (int j = lo + lane; j <= hi; j += 64) sum += double(weight(xr[j] * scale));
         sum = dpp_sum(sum);
         if (sum != sum) {
-            store_nan_row<SO>(yr, lo, hi, kc, lane, 64);
+            store_nan_row<SO>(yr, lo, hi, lane, kc, 64);
             return;
         }
         const float inv = sum == 0.0 ? 0.0f : float(1.0 / sum);
@@ -555,7 +553,7 @@ namespace mg
         // range (capped scores stay below it)
         const bool nan = !(sum < __builtin_huge_valf());
         if (CAP && nan) {
-            store_nan_row<SO>(y + row * a.ldy, int(r.lo64), int(r.hi64), int(a.kc), lane, 64);
+            store_nan_row<SO>(y + row * a.ldy, r.lo64, r.hi64, lane, a.kc, 64);
             return;
         }
         if (!CAP && (nan || !(__builtin_fabsf(mc) < kFastMax))) {
@@ -598,7 +596,7 @@ namespace mg
 #pragma unroll
         for (int i = 0; i < WPR; ++i) L += redd[i];
         if (L != L) {
-            store_nan_row<SO>(y + row * a.ldy, int(r.lo64), int(r.hi64), int(a.kc), int(threadIdx.x), 64 * WPR);
+            store_nan_row<SO>(y + row * a.ldy, r.lo64, r.hi64, threadIdx.x, a.kc, 64 * WPR);
             return;
         }
         fast_store<SO, CH, WPR, VEC>(a, y, row, float(1.0 / L), M == kNegInf, lane, w, r);
@@ -688,13 +686,16 @@ namespace mg
         for (int i = threadIdx.x; i < nch; i += blockDim.x) // a maximum of -inf: a sum of 0 or NaN
             L += pr[i].x == kNegInf ? double(pr[i].y) : double(pr[i].y) * mgm::exp(double(pr[i].x) - double(M));
         L = block_sum_f64(L, redd);
+        if (L != L) { // (the whole work-group)
+            store_nan_row<SO>(yr, lo, hi, base + threadIdx.x, base + kSplitChunk < a.kc ? base + kSplitChunk : a.kc, 256);
+            return;
+        }
         const float inv = M == kNegInf ? 0.0f : float(1.0 / L);
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             const int64_t j0 = base + int64_t(threadIdx.x + 256 * c) * 8;
 #pragma unroll
             for (int e = 0; e < 8; ++e) s[c][e] = s[c][e] == kNegInf ? 0.0f : exp_diff(s[c][e], M) * inv;
-            if (L != L) nan_row8(s[c], j0, lo, hi);
             store_probs<SO>(a, yr, j0, vec, s[c]);
         }
     }
@@ -806,13 +807,16 @@ namespace mg
         for (int i = threadIdx.x; i < nch; i += blockDim.x) // a maximum of -inf: a sum of 0 or NaN
             L += pr[i].x == kNegInf ? pr[i].y : pr[i].y * __builtin_amdgcn_exp2f(pr[i].x - M);
         L = block_sum_dpp(L, red);
+        if (L != L) { // (the whole work-group)
+            store_nan_row<SO>(yr, lo, hi, base + threadIdx.x, base + kSplitChunk < a.kc ? base + kSplitChunk : a.kc, 256);
+            return;
+        }
         const float inv = M == kNegInf ? 0.0f : 1.0f / L;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             const int64_t j0 = base + int64_t(threadIdx.x + 256 * c) * 8;
 #pragma unroll
             for (int e = 0; e < 8; ++e) t[c][e] = t[c][e] == kNegInf ? 0.0f : __builtin_amdgcn_exp2f(t[c][e] - M) * inv;
-            if (L != L) nan_row8(t[c], j0, lo, hi);
             store_probs<SO>(a, yr, j0, vec, t[c]);
         }
     }
