@@ -232,8 +232,9 @@ def test_sample_rows_threshold_bin_on_top(prims):
 
 @pytest.mark.parametrize("temp", (1.0, 0.0))
 def test_sample_rows_split_rows(prims, temp):
-    """rows of V >= 16384 with sorted outputs and no top_k cut run split over
-    several work-groups per row: a fully masked row (the raw argmax), NaN and
+    """rows of V >= 16384 with sorted outputs and no top_k cut run over several
+    work-groups per row (register slices up to 64 rows; the split path's turn is
+    test_sample_rows_split_path): a fully masked row (the raw argmax), NaN and
     -inf entries, a row whose maximum sits in the last slice, and greedy rows
     (temperature 0: np.argmax, NaN counting as the largest) beside sampled ones"""
     import torch
@@ -267,8 +268,8 @@ def test_sample_rows_split_rows(prims, temp):
 
 @pytest.mark.parametrize("V,ld", ((30001, 30001), (40000, 40003), (50000, 50000)))
 def test_sample_rows_split_unaligned(prims, V, ld):
-    """the split path on rows whose slices start off 16-byte boundaries (odd V or
-    row stride: entry-by-entry loads there), and on aligned rows of three rows"""
+    """rows of odd width or stride, off 16-byte boundaries, and three aligned ones
+    (register slices)"""
     import torch
     rows = 3
     wide = O.normal(58, (rows, ld), 0.0, 3.0, F32).view(np.float32).copy()
@@ -292,8 +293,8 @@ def test_sample_rows_split_unaligned(prims, V, ld):
 
 @pytest.mark.parametrize("rows", (64, 100))
 def test_sample_rows_split_fewer_slices(prims, rows):
-    """64 rows split over 4 work-groups each (the bench's shape at a smaller V),
-    100 rows over 2"""
+    """64 rows over 8 register slices each (the bench's shape at a smaller V), 100
+    rows over 2 work-groups of the split path"""
     import torch
     V = 20000
     L = O.normal(59, (rows, V), 0.0, 3.0, F32).view(np.float32).copy()
@@ -320,9 +321,9 @@ def test_sample_rows_split_fewer_slices(prims, rows):
 
 @pytest.mark.parametrize("case", range(8))
 def test_sample_rows_split_random(prims, case):
-    """seeded random configurations through the split path (sorted outputs, no
-    top_k cut): row counts giving 8 down to 2 work-groups per row, widths off
-    whole groups, spreads, -inf and NaN entries, top_p / min_p / temperature;
+    """seeded random configurations over several work-groups a row (sorted outputs, no
+    top_k cut): row counts of 16 and 8 register slices and of the split path's 2
+    work-groups, widths off whole groups, spreads, -inf and NaN entries, top_p / min_p / temperature;
     rows whose cut float32 and f64 place apart are skipped (asserted rare)"""
     import torch
     rng = np.random.default_rng(1000 + case)
@@ -490,6 +491,28 @@ def check_sorted_rows(prims, L, top_p=0.9, temp=1.0, raw=None, ld=None):
         assert np.array_equal(ids[r, :n[r]], wi), r
         assert np.abs(probs[r, :n[r]].astype(np.float64) - wp).max() <= 2e-6, r
     return n
+
+
+@pytest.mark.parametrize("rows,V,ld", ((65, 30000, 30000), (85, 16387, 16389), (128, 20002, 20002), (3, 458753, 458753),
+                                       (9, 460001, 460002)))
+@pytest.mark.parametrize("temp", (1.0, 0.0))
+def test_sample_rows_split_path(prims, rows, V, ld, temp):
+    """the four split kernels: 65 to 128 rows (3 and 2 work-groups a row) and rows too
+    wide for the register slices (8), aligned and not, greedy and sampled: a fully
+    masked row (the raw argmax), NaN and -inf entries, the maximum in the last slice,
+    and equal values past the threshold bin's room"""
+    rng = np.random.default_rng(90 + rows)
+    L = (rng.standard_normal((rows, V)) * 3.5).astype(np.float32)
+    raw = np.argmax(L, axis=1)
+    L[0] = -np.inf
+    L[1, ::7] = np.nan
+    L[2, ::3] = -np.inf
+    L[2, V - 1] = 40.0
+    if rows > 4:
+        L[3] = np.float32(1.0)
+        L[3, rng.permutation(V)[:50]] = rng.uniform(30.0, 33.0, 50).astype(np.float32)
+        L[4, V // 2] = np.nan
+    check_sorted_rows(prims, L, 0.8, temp, raw, ld)
 
 
 @pytest.mark.parametrize("rows,V,sigma", ((1, 17001, 2.5), (20, 17001, 2.5), (1, 32000, 2.75), (20, 32000, 3.0),
