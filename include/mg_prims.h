@@ -217,7 +217,11 @@ int mg_dequant_q8_0(mg_ctx *ctx, const int8_t *qs, const uint16_t *d, void *out,
  * probabilities in the p.v product, the reference tier's contract: a
  * numerical envelope, not bits. head_dim 64 or 128; any number of query heads
  * per kv head. Few query tiles over many keys split their keys over the
- * context's workspace when their partials fit it. */
+ * context's workspace when their partials fit it; a row's output then differs
+ * from the same row in another call by the order of its f32 sums alone (below
+ * 1e-6 of its norm), unless some score passes all of the row's first 64 by more
+ * than 8 ln 2, where bf16 may round its weights elsewhere (inside the envelope
+ * either way). */
 int mg_attn_prefill(mg_ctx *ctx, const uint16_t *q, int64_t ldq, const uint16_t *k_cache, const uint16_t *v_cache,
                     int64_t tokens, int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t cache_slots,
                     int64_t pos0, int64_t window, double scaling, float *out, int64_t ldo);
@@ -248,7 +252,9 @@ int mg_quantize_q8_0(mg_ctx *ctx, const uint16_t *w, int64_t rows, int64_t in, i
  * [batch, in] (row stride ldx, 0 = in), y f32 [batch, rows] (row stride ldy,
  * 0 = rows). blockdot = 0: every weight is bf16(q * d) first (the engine's
  * default, consistent with a prefill that dequantizes); blockdot = 1:
- * sum over blocks of d * sum(q * x) (llama.cpp's dot). f32 accumulation. */
+ * sum over blocks of d * sum(q * x) (llama.cpp's dot). f32 accumulation, in an
+ * order that depends on batch and sizes (dot instructions or the matrix cores):
+ * a row's bits may differ between batches, within the bound either way. */
 int mg_gemv_q8_0(mg_ctx *ctx, const int8_t *qs, const uint16_t *d, const uint16_t *x, int64_t batch, int64_t rows,
                  int64_t in, int64_t ldx, float *y, int64_t ldy, int blockdot);
 

@@ -273,7 +273,8 @@ namespace mg
         }
     }
 
-    // Two to eight activation rows over a weight of 256-quant rows: the weights
+    // Two to eight activation rows over a weight of 256-quant rows (where this is the
+    // faster form, see the launcher): the weights
     // are read and dequantized once for all of them, and the products run on the
     // matrix cores (v_mfma_f32_16x16x32_bf16: A = 16 weight rows, B = the batch
     // padded to 16 columns by its last row, whose columns are not stored). The

@@ -9,10 +9,13 @@
 //   masked keys (causal / window):   excluded, probability exactly 0
 //   p = exp(s - max) / sum           written once at the output dtype
 // The reference evaluates the exponentials and the sum in f64 (twin) or f32
-// (compat, 856-870); here the exponentials are f32 (an accurate exp of the
-// exactly formed s - max) summed in f64 in a fixed order, which keeps p within
-// a few f32 ulp of the f64 value: the bf16 output is within 1 ulp of the
-// twin's and the f32 output within 1e-6 relative.
+// (compat, 856-870). Here f32 and f64 outputs, 16-bit scores and capped rows of
+// more than 2048 keys take f32 exponentials (an accurate exp of the exactly formed
+// s - max) summed in f64 in a fixed order, which keeps p within a few f32 ulp of
+// the f64 value; f32 scores to 16-bit probabilities otherwise take the hardware
+// exp2, in f32 sums up to 2048 keys and f64 or chunked ones beyond, a few 1e-7
+// relative. 16-bit outputs are within 1 ulp of the twin's, f32 ones within 1e-6
+// relative.
 //
 // Rows of up to 2048 keys: one wave per row (the fast path runs one-wave
 // work-groups), the row in registers (8 keys per lane per chunk), one read
@@ -938,12 +941,12 @@ namespace mg
                 // log2-domain factor: the scale folds in unless the cap comes after it
                 const float c2 = float((CAP ? 1.0 : double(a.scale)) * 1.4426950408889634);
                 const unsigned wgs = unsigned(a.nrows); // < 2^31: checked above
-                // Without the cap the kernel needs few registers (8 waves per SIMD
-                // would fit) but streams fastest at 4: the LDS each work-group
+                // Without the cap the kernel needs few registers (55: 9 waves per
+                // SIMD would fit) but streams fastest at 5: the LDS each work-group
                 // reserves (and never touches) holds a CU at 20 of them (measured
                 // with four keys per lane and load: 110.5 us at 8 waves, 109.9 at
-                // 4, 109.0 at 5, 126.4 at 3, config 4). With the cap its
-                // registers allow 5, which the extra arithmetic uses.
+                // 4, 109.0 at 5, 126.4 at 3, 40 heads of 2048 by 2048). With the cap
+                // its registers (89) allow 5, which the extra arithmetic uses.
                 const unsigned lds = CAP ? 0u : kLdsPerCu / (4u * kFastWavesNoCap);
                 auto go = [&](auto kern) {
                     hipLaunchKernelGGL(kern, dim3(wgs), dim3(64), lds, c->stream, xi, yo, a, c2);
@@ -979,10 +982,11 @@ namespace mg
                 const float c2 = float((CAP ? 1.0 : double(a.scale)) * 1.4426950408889634);
                 // as in k_softmax_fast, a reserved and untouched part of the LDS
                 // holds the waves per SIMD where the row streams best: 4 for
-                // vector rows of two waves (40 000 rows of 4000: 143 us against
-                // 161 unheld, 150 at 5, 159 at 6), 6 for the others (10 000 of
-                // 16 000: 158 against 162, 159 at 4; 28 000 of 5003: 145 against
-                // 149, 155 at 4)
+                // vector rows of two waves (40 000 rows of 4000: 145 us against
+                // 160 unheld, 152 at 5, 157 at 6), 6 for the others (13 720 of
+                // 12 000: 159 against 164, 172 at 4; 32 960 of 5003: 164 against
+                // 169, 175 at 4). Over 14 lengths from 2049 to 16384 and 40 to
+                // 40 000 rows both lie within 5 % of the best of 3 to 8 and none.
                 auto go = [&](auto kern, unsigned waves) {
                     const unsigned hold = vec && waves == 2 ? 4u : 6u;
                     const unsigned lds = CAP ? 0u : (kLdsPerCu - 8192u) * waves / (4u * hold);

@@ -64,13 +64,13 @@ def test_shapes(prims, nq, nkv, D):
 @pytest.mark.parametrize("hpg", (1, 2, 3, 4, 5, 6, 8))
 @pytest.mark.parametrize("D", (64, 128))
 def test_group_sizes(prims, hpg, D):
-    """every query-head count per KV head (one wave per head of the group)"""
+    """query-head counts per KV head: pairs of a wave mix rows and heads"""
     prefill_case(prims, 70, 2 * hpg, 2, D, 80, 0, seed=110 + hpg)
 
 
 @pytest.mark.parametrize("hpg", (9, 10, 16))
 def test_large_groups(prims, hpg):
-    """groups past 8 heads over several work-groups (9 -> 3 x 3, 10 -> 2 x 5, 16 -> 2 x 8)"""
+    """groups past 8 heads (a window's key steps start by groups of 3 x 3, 2 x 5, 2 x 8)"""
     prefill_case(prims, 70, 2 * hpg, 2, 128, 80, 0, seed=160 + hpg)
 
 
@@ -99,7 +99,7 @@ def test_window_ring_many_steps(prims):
 
 
 def test_short_and_ragged(prims):
-    """one row, rows that end inside a 16-row tile, a 32-row tile boundary"""
+    """one row, and row counts about a wave's 32 pairs and a tile's 128"""
     for T in (1, 15, 17, 31, 32, 33):
         prefill_case(prims, T, 8, 2, 128, 64, 0, seed=130 + T)
 
